@@ -17,6 +17,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "internal.h"
 
 namespace hn {
@@ -333,6 +335,7 @@ struct RowsArgs {
   float scale;
   FFTAxis ax;
   int lgL;
+  int lgQ;  // adjoint: 2^lgQ transforms of an image side by side in a workgroup
 };
 
 // image rows -> deconvolve * scale (* smap) -> pad -> FFT -> grid rows
@@ -441,16 +444,27 @@ __global__ __launch_bounds__(kThreads) void k_rows_fwd(RowsArgs a) {
 
 // grid rows -> FFT -> crop -> deconvolve * scale (* conj smap, summed over the
 // chunk's coils of one batch) -> image rows
+//
+// A workgroup's 2^lgL lines are 2^(lgL - lgQ) image rows of 2^lgQ transforms
+// each: with many rows a workgroup walks the coils of its rows one by one
+// (lgQ = 0), with few rows (2D images) that serial walk on a few workgroups
+// is all there is to see -- 32 workgroups for 256 rows, each waiting for one
+// coil's loads, FFT and maps after the other -- so the coils go side by side
+// and their sums meet in LDS at the end, in coil order.  Measured with
+// lgQ = 0 against the rule of rows_adj(): 256^2, 8 coils 47.6 -> 10.3 us,
+// 16 coils 89 -> 17; 320^2, 32 coils 233 -> 71; 192^2, 12 frames of 8 coils
+// 43 -> 29.
 template <int S, int EPT, int FIX = 0, int FLGL = 0>
 __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   extern __shared__ float2 buf[];
   // FIX > 0: FIX-point rows, 2^FLGL per workgroup, passes fixed at compile time
   if constexpr (FIX > 0) a.lgL = FLGL;
   const int L = 1 << a.lgL, LP = L + 1;
+  const int lgR = a.lgL - a.lgQ, R = 1 << lgR, Q = 1 << a.lgQ;
   const float2* twl = stage_twiddles(buf, a.ax, LP);
   const int rows = a.M0 * a.M1;
   const BlockIdx3 bi = remapped_block();
-  const int r0 = bi.x * L;
+  const int r0 = bi.x * R;
   const int n = a.nf2;
   const int64_t N = (int64_t)rows * a.M2;
   // one output image per image present in the chunk, the sum of its
@@ -461,28 +475,33 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   const int te = min(a.t0 + a.T, (out_img + 1) * per_img);
   const bool add_existing = tb % per_img != 0;
   // line-major thread mapping: thread (l, x0) handles positions x0 + j * TPL
-  // of line l, so it keeps one row base across the coil loop
+  // of line l (row l / Q, transform l % Q of the Q), so it keeps one row base
+  // across the coil loop
   const int TPL = kThreads >> a.lgL;  // threads per line (n <= TPL * EPT)
   const int l = threadIdx.x / TPL, x0 = threadIdx.x - l * TPL;
-  const int r = r0 + l;
+  const int q = l & (Q - 1);
+  const int r = r0 + (l >> a.lgQ);
   const bool rok = r < rows;
   int64_t grow = 0;
   if (rok) {
     const int i0 = r / a.M1, i1 = r - i0 * a.M1;
     grow = ((int64_t)kept_pos(i0, a.M0, a.nf0) * a.nf1 + kept_pos(i1, a.M1, a.nf1)) * n;
   }
-  // coil sum of the cropped lines in LDS after the line data and twiddles;
-  // each entry is only touched by the thread that owns it
-  float2* accl = buf + (size_t)n * (LP + 1) + (size_t)l * a.M2;
+  // sum of the line's transforms, cropped, in LDS after the line data and
+  // twiddles; each entry is only touched by the thread that owns it
+  float2* acc0 = buf + (size_t)n * (LP + 1);
+  float2* accl = acc0 + (size_t)l * a.M2;
 
-  for (int tt = tb; tt < te; ++tt) {
+  for (int tg = tb; tg < te; tg += Q) {
+    const int tt = min(tg + q, te - 1);
+    const bool tok = rok && tg + q < te;
     const float2* g = a.grid + (int64_t)(tt - a.t0) * a.gstride + grow;
     {
       float2 v[EPT];
 #pragma unroll
       for (int j = 0; j < EPT; ++j) {
         const int x = x0 + j * TPL;
-        v[j] = (rok && x < n) ? g[x] : make_float2(0.f, 0.f);
+        v[j] = (tok && x < n) ? g[x] : make_float2(0.f, 0.f);
       }
 #pragma unroll
       for (int j = 0; j < EPT; ++j) {
@@ -520,7 +539,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
       const int x = x0 + j * TPL;
       if (x < a.M2) {
         float2 v = make_float2(0.f, 0.f);
-        if (rok) {
+        if (tok) {
           v = buf[kept_pos(x, a.M2, n) * LP + l];
           if (sm) {
             float2 s2 = FIX > 0 ? sv[j] : sm[x];
@@ -532,17 +551,24 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
             v = cmul(v, cv);
           }
         }
-        accl[x] = (tt == tb) ? v : cadd(accl[x], v);
+        accl[x] = (tg == tb) ? v : cadd(accl[x], v);
       }
     }
     __syncthreads();
   }
-  if (!rok) return;
-  const int i0 = r / a.M1, i1 = r - i0 * a.M1;
+  // thread (row, x1) sums the Q lines of its row in transform order
+  const int TPR = kThreads >> lgR;
+  const int ro = threadIdx.x / TPR, x1 = threadIdx.x - ro * TPR;
+  const int rr = r0 + ro;
+  if (rr >= rows) return;
+  const int i0 = rr / a.M1, i1 = rr - i0 * a.M1;
   const float rs = a.dec0[i0] * a.dec1[i1] * a.scale;
-  float2* dst = a.img_out + (int64_t)out_img * N + (int64_t)r * a.M2;
-  for (int x = x0; x < a.M2; x += TPL) {
-    float2 v = cscale(accl[x], rs * a.dec2[x]);
+  const float2* accr = acc0 + (size_t)(ro << a.lgQ) * a.M2;
+  float2* dst = a.img_out + (int64_t)out_img * N + (int64_t)rr * a.M2;
+  for (int x = x1; x < a.M2; x += TPR) {
+    float2 v = accr[x];
+    for (int k = 1; k < Q; ++k) v = cadd(v, accr[(size_t)k * a.M2 + x]);
+    v = cscale(v, rs * a.dec2[x]);
     if (add_existing) v = cadd(v, dst[x]);
     dst[x] = v;
   }
@@ -1083,7 +1109,13 @@ int rows_adj(const hipnufft_plan_s* p, float2* img, const float2* smaps, int C, 
   const int L = p->fft[2].L;
   const int per_img = (smaps ? C : 1) * nmaps;
   const int nimg = (t0 + T - 1) / per_img - t0 / per_img + 1;
-  const dim3 grd((unsigned)((rows + L - 1) / L), (unsigned)nimg);
+  // transforms of an image side by side while the rows alone give fewer than
+  // two workgroups per CU (each then walks fewer coils)
+  while ((1 << a.lgQ) < L && (1 << a.lgQ) < std::min(per_img, T) &&
+         (int64_t)((rows * (int64_t)(1 << a.lgQ) + L - 1) / L) * nimg < 512)
+    ++a.lgQ;
+  const int R = L >> a.lgQ;
+  const dim3 grd((unsigned)((rows + R - 1) / R), (unsigned)nimg);
   const size_t lds = rows_adj_lds(p->fft[2], a.M2);
   StageScope timer(p, kStageRowsAdj);
   const FFTAxis& ax = p->fft[2];
