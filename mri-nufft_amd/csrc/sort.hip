@@ -324,6 +324,8 @@ __global__ __launch_bounds__(kThreads) void k_sub_emit(const int32_t* bs, const 
     st[soff[b] + s] = (int32_t)b;
     sb[soff[b] + s] = bs[b] + s * S;
   }
+  // the items' points follow each other: an item ends where the next begins
+  if (b == nkeys - 1) sb[soff[b] + k] = bs[nkeys];
 }
 
 // spread work items per tile: 1 for light tiles (also empty ones: every tile
@@ -737,7 +739,7 @@ int build_points(hipnufft_plan_s* p, int nsets, const int64_t* Ms, const float* 
     if (nsub > p->sub_cap || !p->sub_tile) {
       int64_t c1 = 0, c2 = 0;
       if ((rc = grow(&p->sub_tile, &c1, nsub))) return rc;
-      if ((rc = grow(&p->sub_begin, &c2, nsub))) return rc;
+      if ((rc = grow(&p->sub_begin, &c2, nsub + 1))) return rc;
       p->sub_cap = c1;
     }
     p->nsub = nsub;

@@ -65,7 +65,7 @@ struct SpreadArgs {
 struct InterpArgs {
   PtsGeom g;
   const int32_t* sub_tile;  // key (set * nbins + tile) per work item
-  const int32_t* sub_begin;
+  const int32_t* sub_begin;  // first point per work item; then the number of points
   const int32_t* bin_start;
   int max_sub;
   int sub0;                 // first work item of the launch
@@ -93,8 +93,8 @@ struct InterpArgs {
   int mask_stage;    // stage only the chunks the points read (needs grid_bytes)
   int grid_bytes;    // bytes of one transform's grid, < 2^31
   const uint16_t* sub_mask;  // per work item and region row: the chunks read
-  int lds_pad;               // k_interp_stream: LDS cells after each region row
-  uint32_t lds_row_mag;      // and the magic multiplier of the padded row length
+  uint32_t lds_row_mag;      // k_interp_stream, k_interp_pairs: magic multiplier of the
+  uint32_t lds_plane_mag;    // LDS row length and plane stride
 };
 
 // dword 3 of a raw buffer resource on gfx9-family GPUs (gfx950 included):
@@ -1210,6 +1210,11 @@ __device__ __forceinline__ int wrap_coord(int x, int nfd, int wrap1) {
   return x;
 }
 
+__device__ __forceinline__ int wrap_once(int x, int nfd) {  // x inside [-nf, 2nf)
+  x += x < 0 ? nfd : 0;
+  return x >= nfd ? x - nfd : x;
+}
+
 // Stage the tile + halo region of transforms [t0, t0 + G) into LDS: cell
 // (gg, l_0, .., l_{D-1}) at gg * RC + row-major l.  In 2D and 3D the region
 // is NR rows of RL cells along the last axis: a table after the staged
@@ -1465,18 +1470,23 @@ __device__ __forceinline__ void stage_region_masked(const InterpArgs& a, float2*
 }
 
 
+// region cell along axis d of a footprint that starts at grid cell `cell`
+template <int D>
+__device__ __forceinline__ int region_cell(const InterpArgs& a, int cell, int d, const int* rorg) {
+  int l = cell - rorg[d];
+  if (l < 0) l += a.g.nf[d];
+  if (l >= a.g.nf[d]) l -= a.g.nf[d];
+  // memory safety; a sorted point always satisfies it
+  return min(max(l, 0), (d == D - 1 ? a.span : 1) * a.g.tile[d]);
+}
+
 template <int D, int W>
 __device__ __forceinline__ void point_setup(const InterpArgs& a, int p, const int* rorg,
                                             int* ls, float (*wt)[W]) {
   const float inv_hw = 2.0f / W;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    int l = a.g.cell[d][p] - rorg[d];
-    if (l < 0) l += a.g.nf[d];
-    if (l >= a.g.nf[d]) l -= a.g.nf[d];
-    // memory safety; a sorted point always satisfies it
-    l = min(max(l, 0), (d == D - 1 ? a.span : 1) * a.g.tile[d]);
-    ls[d] = l;
+    ls[d] = region_cell<D>(a, a.g.cell[d][p], d, rorg);
     const float off = a.g.off[d][p];
 #pragma unroll
     for (int j = 0; j < W; ++j) wt[d][j] = es_eval(off - (float)j, inv_hw, a.g.beta);
@@ -1631,15 +1641,13 @@ __global__ __launch_bounds__(NT, 4) void k_interp(InterpArgs a) {
 // interpolation in 5.5 ms; 1024 threads with two buffers in 6.6 ms; 512
 // with two, one workgroup per CU, 7.1 ms), region cells a buffer holds
 // (8 x 8 x 16 tiles, two along the last axis, w <= 8), region rows the row
-// tables hold, the widest kernel it is built for (its footprint loops unroll
-// fully) and the LDS cells after each region row (rows of 41 or 42 cells
-// measured the same as 39, rows of 40 slower)
+// tables hold and the widest kernel it is built for (its footprint loops
+// unroll fully)
 constexpr int kStreamNT = 512;
 constexpr int kStreamNB = 1;
 constexpr int kStreamCells = 9728;
 constexpr int kStreamRows = 256;
 constexpr int kStreamMaxW = 8;
-constexpr int kStreamPad = 0;
 // 2D regions (32 x 32 tiles plus the halo: 1521 cells) are small, so 2D
 // workgroups of 256 threads hold 2048 cells and several share a CU
 constexpr int kStream2NT = 256;
@@ -1663,14 +1671,31 @@ constexpr int kStream2Rows = 128;
 // the item allows; it holds at most NT >> LGMIN points), lane s summing
 // the kernel rows j0 = s, s + lp, ...; the partial sums meet by lane
 // exchanges in a fixed order, so the result does not depend on the run.
-// The footprint gathers bound the kernel: random 16-byte LDS reads.
-template <int D, int W, int NT, int NB, int CELLS, int ROWS>
+//
+// PAIR: the footprint gathers bound the kernel, and LDS serves 16-byte reads
+// at 16-byte addresses about twice as fast as the 8-byte reads that a
+// footprint starting at any cell needs (a microbenchmark of this pattern: 88
+// to 115 against 62 bytes per clock and CU).  The region then starts at an
+// even grid cell and its rows hold an even number of cells, so a row's cells
+// are read as the aligned pairs that cover [start, start + W): one cell more
+// than the footprint, which is replaced by zero before its (zero) weight --
+// it belongs to no footprint and may hold anything.  A pair never straddles
+// a 16-cell chunk, a tile or the grid's end, so the region also moves in
+// 16-byte pieces, a quarter of the loads and of the offsets held.  Needs an
+// even last axis, an even tile and 16-byte aligned grids: every grid of a
+// full plan; spread / interp-only plans on odd axes keep single cells.
+template <int D, int W, int NT, int NB, int CELLS, int ROWS, bool PAIR>
 __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
   // static LDS (NB buffers of CELLS cells and the row tables): the compiler
   // then knows how many workgroups share a CU
-  __shared__ float2 lds[NB * CELLS + ROWS];
-  constexpr int K = 2 * CELLS / NT;  // staged words per thread
+  __shared__ __attribute__((aligned(16))) float2 lds[NB * CELLS + ROWS];
+  constexpr int PW = PAIR ? 4 : 1;  // 32-bit words per staged piece
+  constexpr int K = (2 * CELLS + PW * NT - 1) / (PW * NT);  // staged pieces per thread
   constexpr int DL = D - 1;                 // the contiguous axis
+  constexpr int SH = PAIR ? (W / 2) & 1 : 0;  // cells the region starts earlier (tiles are even)
+  // pairs that cover a row of W cells from any start (cells 0 .. W of them)
+  constexpr int NP = (W + 2) / 2;
+  constexpr int NC = PAIR ? W + 1 : W;  // cells of a row that may carry a weight
   constexpr uint32_t kSkip = 0x80000000u;
   constexpr int LGMIN = NT >= 1024 ? 1 : 0;  // items hold at most NT >> LGMIN points
   constexpr int KJ = (W + (1 << LGMIN) - 1) >> LGMIN;  // rows per lane at the fewest lanes
@@ -1686,9 +1711,10 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
   int rorg[3], R[3];
   region_of<D, W>(a, tile, rorg, R);
   const int NR = D == 3 ? R[0] * R[1] : R[0];  // region rows along the contiguous axis
-  const int RL = R[DL] + a.lds_pad;  // LDS row length: the padding moves rows across banks
+  rorg[DL] -= SH;
+  const int RL = PAIR ? (R[DL] + SH + 1) & ~1 : R[DL];  // LDS row length
   const int RC = NR * RL;
-  const int RCP = (RC + 31) & ~31;  // a buffer: whole 64-word wave segments
+  const int RCP = (RC + 32 * PW - 1) & ~(32 * PW - 1);  // a buffer: whole segments of 64 pieces
   const int tid = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -1707,19 +1733,21 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
     rowmask[r] = a.sub_mask ? (uint32_t)a.sub_mask[(int64_t)sub * NR + r] : 0xffffffffu;
   }
   __syncthreads();
-  const int phase = ((rorg[DL] % 16) + 16) % 16;
+  // chunk of region cell z: (z + phase) / 16 of the row's mask, whose cell 0
+  // is region cell SH
+  const int phase = (((rorg[DL] + SH) % 16) + 16) % 16 - SH;
   uint32_t off[K];
 #pragma unroll
   for (int u = 0; u < K; ++u) {
-    const int wd = tid + u * NT;  // word: cell wd / 2, real (0) or imaginary (1) part
-    const int c = wd >> 1;
+    const int pc = tid + u * NT;  // a pair of cells, or one 32-bit word of a cell
+    const int c = PAIR ? 2 * pc : pc >> 1;
     off[u] = kSkip;
     if (c < RC) {
       const int r = mdiv(c, a.lds_row_mag);
       const int z = c - r * RL;
-      if (z < R[DL] && ((rowmask[r] >> ((z + phase) >> 4)) & 1u))
+      if ((rowmask[r] >> ((z + phase) >> 4)) & 1u)
         off[u] = (uint32_t)(rowoff[r] + wrap_coord(rorg[DL] + z, a.g.nf[DL], a.wrap1)) * 8u +
-                 4u * (uint32_t)(wd & 1);
+                 (PAIR ? 0u : 4u * (uint32_t)(pc & 1));
     }
   }
 
@@ -1732,21 +1760,31 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
   const int s = tid & (lp - 1);
   const bool live = p < pe;
   int lbase = 0;  // the lane's first footprint row j0 = s, as an LDS cell index
-  float wt1[W], wt2[W], w0[KJ];
+  float wt1[W], wt2[NC], w0[KJ];
+  bool odd = false;  // PAIR: the footprint starts at the second cell of a pair
   int64_t kbase = 0, kstep = 0;  // k-space offset of transform t: kbase + t * kstep
   float dens = 1.0f;
 #pragma unroll
-  for (int j = 0; j < W; ++j) wt1[j] = wt2[j] = 0.0f;
+  for (int j = 0; j < W; ++j) wt1[j] = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NC; ++j) wt2[j] = 0.0f;
 #pragma unroll
   for (int k = 0; k < KJ; ++k) w0[k] = 0.0f;
   if (live) {
     int ls[3];
     float wt[D][W];
+    rorg[DL] += SH;
     point_setup<D, W>(a, p, rorg, ls, wt);
+    ls[DL] += SH;
+    odd = PAIR && (ls[DL] & 1);
+    if (PAIR) ls[DL] &= ~1;
 #pragma unroll
-    for (int j = 0; j < W; ++j) {  // wt2: the contiguous axis; wt1: the middle one (3D)
-      wt1[j] = wt[D == 3 ? 1 : 0][j];
-      wt2[j] = wt[DL][j];
+    for (int j = 0; j < W; ++j) wt1[j] = wt[D == 3 ? 1 : 0][j];  // the middle axis (3D)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {  // the contiguous axis
+      const float even_w = j < W ? wt[DL][j < W ? j : 0] : 0.0f;
+      const float odd_w = j > 0 ? wt[DL][j > 0 ? j - 1 : 0] : 0.0f;
+      wt2[j] = odd ? odd_w : even_w;
     }
     const float inv_hw = 2.0f / W;
     const float off0 = a.g.off[0][p];
@@ -1761,8 +1799,8 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
   }
   const int rstep = lp * (D == 3 ? R[1] : 1) * RL;  // LDS cells between the lane's rows
 
-  // the region of transform t into buffer b: load u of wave w fills words
-  // [u NT + 64 w, u NT + 64 w + 64) of the buffer
+  // the region of transform t into buffer b: load u of wave w fills the 64
+  // pieces from u NT + 64 w of the buffer
   auto stage = [&](int t, int b) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.grid + (int64_t)(tb + t) * a.grid_stride), (short)0, a.grid_bytes,
@@ -1770,10 +1808,40 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
     float* buf = reinterpret_cast<float*>(lds + b * RCP);
 #pragma unroll
     for (int u = 0; u < K; ++u) {
-      const int w0d = u * NT + wave * 64;  // uniform
+      const int w0d = (u * NT + wave * 64) * PW;  // uniform
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass rejects the 16-byte form
       if (w0d < 2 * RCP)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (__attribute__((address_space(3))) void*)(buf + w0d), 4, off[u], 0, 0, 0);
+            rs, (__attribute__((address_space(3))) void*)(buf + w0d), 4 * PW, off[u], 0, 0, 0);
+#endif
+    }
+  };
+  // sum over one footprint row: its reads first, so that they are in flight
+  // together (read one by one, each waited for its predecessor's result:
+  // 4.52 -> 4.41 ms for the 16-coil 192^3 interpolation)
+  auto row_sum = [&](const float2* row, float& rx, float& ry) {
+    float2 c[2 * NP];
+    if constexpr (PAIR) {
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        const float4 v = reinterpret_cast<const float4*>(row)[q];
+        c[2 * q] = make_float2(v.x, v.y);
+        c[2 * q + 1] = make_float2(v.z, v.w);
+      }
+      // the cell outside the footprint
+      c[0].x = odd ? 0.0f : c[0].x;
+      c[0].y = odd ? 0.0f : c[0].y;
+      c[W].x = odd ? c[W].x : 0.0f;
+      c[W].y = odd ? c[W].y : 0.0f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < W; ++j) c[j] = row[j];
+    }
+    rx = ry = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      rx += wt2[j] * c[j].x;
+      ry += wt2[j] * c[j].y;
     }
   };
   if (NB == 2) stage(0, 0);
@@ -1805,29 +1873,13 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
         if constexpr (D == 3) {
 #pragma unroll
           for (int j1 = 0; j1 < W; ++j1) {
-            // the row's reads first, so that they are in flight together
-            // (read one by one, each waited for its predecessor's result:
-            // 4.52 -> 4.41 ms for the 16-coil 192^3 interpolation)
-            const float2* row = rowk + j1 * RL;
-            float2 c[W];
-#pragma unroll
-            for (int j2 = 0; j2 < W; ++j2) c[j2] = row[j2];
-            float rx = 0.f, ry = 0.f;
-#pragma unroll
-            for (int j2 = 0; j2 < W; ++j2) {
-              rx += wt2[j2] * c[j2].x;
-              ry += wt2[j2] * c[j2].y;
-            }
+            float rx, ry;
+            row_sum(rowk + j1 * RL, rx, ry);
             px += wt1[j1] * rx;
             py += wt1[j1] * ry;
           }
         } else {  // 2D: row s + k lp of the footprint is one line along the contiguous axis
-#pragma unroll
-          for (int j2 = 0; j2 < W; ++j2) {
-            const float2 c = rowk[j2];
-            px += wt2[j2] * c.x;
-            py += wt2[j2] * c.y;
-          }
+          row_sum(rowk, px, py);
         }
         sx += w0[k] * px;
         sy += w0[k] * py;
@@ -1845,6 +1897,263 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
         a.out[(int64_t)(t0 + gg) * a.g.M + p] = r;
       } else {
         a.out[kbase + (t0 + gg) * kstep] = r;
+      }
+    }
+  }
+}
+
+// k_interp_stream for 3D regions of aligned pairs and items of at most 128
+// points: the default of 3D plans.  The footprint gathers bound it, LDS
+// reads and the multiply-adds on them about equally, so both are laid out
+// for the hardware:
+// - every point is spread over 8 lanes, lane s reading the footprint plane
+//   j0 = s, in two trips of 64 points.  16-byte LDS reads are served in
+//   groups of 8 lanes, {0-3, 20-23}, {4-7, 16-19}, {8-11, 28-31} and
+//   {12-15, 24-27} of each half wave; a point's lanes are one such group and
+//   the region's planes lie 4 cells modulo 8 apart, so that a group's reads
+//   meet no bank twice and even the two groups served together rarely do: 25
+//   cycles per row read of a wave in a microbenchmark, against 37 with
+//   points on consecutive lanes and unpadded planes, and 64 for single cells;
+// - the sums over a row run over its pairs without looking at the one cell
+//   that lies outside the footprint (its weight is zero).  That cell may
+//   hold anything, so a sum that comes out not finite is formed again over
+//   the footprint's own cells: selecting zero for it in every row costs 4 of
+//   26 instructions;
+// - the lanes' sums meet by DPP and one swizzle rather than through LDS.
+// - what a workgroup needs before its first region is loaded at once, and an
+//   item's points end where the next item's begin (no look-up of its bins).
+// 192^3, 16 coils, 2.1 M radial samples: single cells 4.46 ms, pairs with
+// points on 1 to 8 consecutive lanes 3.53 ms, this kernel 2.91 ms.  Of those
+// the set-up takes 0.24; without its gathers the kernel takes 2.47, without
+// its loads 2.27.
+constexpr int kPairNT = 512;
+constexpr int kPairCells = 9216;  // two workgroups per CU
+constexpr int kPairTrips = 2;
+constexpr int kPairPoints = kPairTrips * kPairNT / 8;
+
+// cells between the region's planes: at least the plane, 4 modulo 8
+__host__ __device__ __forceinline__ int pair_plane_stride(int plane) {
+  return plane + ((12 - plane % 8) % 8);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                           0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
+// sum over the 8 lanes of a point (see k_interp_pairs): lane s of the eight
+// is s ^ 1, s ^ 2 and s ^ 4 away at lanes l ^ 1, l ^ 2 and l ^ 20
+__device__ __forceinline__ float point_sum(float x) {
+  x = dpp_add<0xB1>(x);
+  x = dpp_add<0x4E>(x);
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x),
+                                                                   0x1f | (20 << 10)));
+}
+
+template <int W>
+__global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
+  constexpr int NT = kPairNT, T = kPairTrips;
+  __shared__ __attribute__((aligned(16))) float2 lds[kPairCells + kStreamRows];
+  constexpr int K = (kPairCells / 2 + NT - 1) / NT;  // staged pairs per thread
+  constexpr int SH = (W / 2) & 1;    // the region starts at an even cell
+  constexpr int NP = (W + 2) / 2;    // pairs that cover a row from any start
+  constexpr int NC = W + 1;          // cells of a row that may carry a weight
+  constexpr uint32_t kSkip = 0x80000000u;
+  const int sub = a.sub0 + (int)xcd_remap(blockIdx.x, gridDim.x);
+  const int key = a.sub_tile[sub];
+  const int set = key / a.g.nbins;
+  const int tile = key - set * a.g.nbins;
+  const int pb = a.sub_begin[sub], pe = a.sub_begin[sub + 1];
+  const int t0 = blockIdx.y * a.G;
+  const int G = min(a.G, a.ts - t0);
+  const int tb = (set - a.k0) * a.ts + t0;  // chunk transform of the first handled here
+  int rorg[3], R[3];
+  region_of<3, W>(a, tile, rorg, R);
+  const int NR = R[0] * R[1];
+  const int RL = (R[2] + SH + 1) & ~1;
+  const int plane = R[1] * RL, PS = pair_plane_stride(plane);
+  const int RCP = (R[0] * PS + 127) & ~127;  // whole segments of 64 pairs
+  const int tid = (int)threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // lane -> (point of the wave's 8, footprint plane s)
+  const int q32 = tid & 31, hi = q32 >> 4;
+  const int s = (q32 & 3) | (hi << 2);
+  const int slot = (((q32 >> 2) & 3) ^ hi) + 4 * ((tid >> 5) & 1);
+  const int n = pe - pb;
+
+  // the points, read before anything waits
+  int cell[T][3], idx[T];
+  float poff[T][3];
+  bool live[T];
+#pragma unroll
+  for (int tr = 0; tr < T; ++tr) {
+    const int p = pb + tr * (NT / 8) + wave * 8 + slot;
+    live[tr] = p < pe && s < W;
+    const int pl = live[tr] ? p : pb;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      cell[tr][d] = a.g.cell[d][pl];
+      poff[tr][d] = a.g.off[d][pl];
+    }
+    idx[tr] = a.g.idx[pl];
+  }
+  const int64_t so = a.g.set_off[set];
+  const int64_t kstep = a.g.set_off[set + 1] - so;  // k-space offset between transforms
+
+  // per region row: wrapped grid offset of its first cell, chunk mask
+  int2* rowtab = reinterpret_cast<int2*>(lds + RCP);
+  for (int r = tid; r < NR; r += NT) {
+    const int l0 = mdiv(r, a.rmag[1]);
+    const int l1 = r - l0 * R[1];
+    rowtab[r] = make_int2((wrap_once(rorg[0] + l0, a.g.nf[0]) * a.g.nf[1] +
+                           wrap_once(rorg[1] + l1, a.g.nf[1])) * a.g.nf[2],
+                          a.sub_mask ? (int)a.sub_mask[(int64_t)sub * NR + r] : 0xffff);
+  }
+  __syncthreads();
+  // chunk of region cell z: (z + phase) / 16 of the row's mask
+  const int phase = (rorg[2] & 15) - SH;
+  uint32_t off[K];
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    const int c = 2 * (tid + u * NT);
+    const int l0 = mdiv(c, a.lds_plane_mag);
+    const int e = c - l0 * PS;
+    const int l1 = mdiv(e, a.lds_row_mag);
+    const int z = e - l1 * RL;
+    const bool in = l0 < R[0] && l1 < R[1];
+    const int2 rt = rowtab[in ? l0 * R[1] + l1 : 0];
+    const int g = rt.x + wrap_once(rorg[2] - SH + z, a.g.nf[2]);
+    off[u] = in && ((rt.y >> ((z + phase) >> 4)) & 1) ? (uint32_t)g * 8u : kSkip;
+  }
+
+  float wt1[T][W], wt2[T][NC], w0[T];
+  int lbase[T];   // LDS cell of the lane's plane at the footprint's first pair
+  bool odd[T];
+  int64_t kbase[T];  // k-space offset of transform t: kbase + t * kstep
+  float dens[T];
+  // lane s of a point evaluates its weights at cell s; the eight meet in the
+  // LDS that the regions take over afterwards
+  constexpr int kWRow = 20;  // floats per point: axis 1 at 0, axis 2 at 8
+  float* wtab = reinterpret_cast<float*>(lds) + (wave * 8 + slot) * kWRow;
+#pragma unroll
+  for (int tr = 0; tr < T; ++tr) {
+    int ls[3];
+    float wd[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      ls[d] = region_cell<3>(a, cell[tr][d], d, rorg);
+      wd[d] = es_eval(poff[tr][d] - (float)s, 2.0f / W, a.g.beta);
+    }
+    ls[2] += SH;
+    odd[tr] = ls[2] & 1;
+    lbase[tr] = (ls[0] + min(s, W - 1)) * PS + ls[1] * RL + (ls[2] & ~1);
+    w0[tr] = wd[0];
+    wtab[tr * (NT / 8) * kWRow + s] = wd[1];
+    wtab[tr * (NT / 8) * kWRow + 8 + s] = wd[2];
+    dens[tr] = (a.mode == 1 && a.density) ? a.density[idx[tr]] : 1.0f;
+    kbase[tr] = a.ts * so + (idx[tr] - so);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int tr = 0; tr < T; ++tr) {
+    const float4* wr = reinterpret_cast<const float4*>(wtab + tr * (NT / 8) * kWRow);
+    const float4 a0 = wr[0], a1 = wr[1], b0 = wr[2], b1 = wr[3];
+    const float wy[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    const float wz[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+    for (int j = 0; j < W; ++j) wt1[tr][j] = wy[j];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const float even_w = j < W ? wz[j < W ? j : 0] : 0.0f;
+      const float odd_w = j > 0 ? wz[j > 0 ? j - 1 : 0] : 0.0f;
+      wt2[tr][j] = odd[tr] ? odd_w : even_w;
+    }
+  }
+  __syncthreads();
+
+  for (int gg = 0; gg < G; ++gg) {
+    if (gg > 0) __syncthreads();  // every lane is done with transform gg - 1
+    float2 y[T];  // the residual's observation
+#pragma unroll
+    for (int tr = 0; tr < T; ++tr) {
+      y[tr] = make_float2(0.f, 0.f);
+      if (a.mode == 1 && live[tr] && s == 0) y[tr] = a.obs[kbase[tr] + (t0 + gg) * kstep];
+    }
+    {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(a.grid + (int64_t)(tb + gg) * a.grid_stride), (short)0, a.grid_bytes,
+          kBufferWord3);
+      // load u of wave w fills the 64 pairs from u NT + 64 w
+#pragma unroll
+      for (int u = 0; u < K; ++u) {
+        const int c0 = 2 * (u * NT + wave * 64);  // uniform
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass rejects the 16-byte form
+        if (c0 < RCP)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              rs, (__attribute__((address_space(3))) void*)(lds + c0), 16, off[u], 0, 0, 0);
+#endif
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+#pragma unroll
+    for (int tr = 0; tr < T; ++tr) {
+      if (tr * (NT / 8) + wave * 8 >= n) continue;  // uniform
+      float sx = 0.f, sy = 0.f;
+      if (live[tr]) {
+        const float2* pl = lds + lbase[tr];
+#pragma unroll
+        for (int j1 = 0; j1 < W; ++j1) {
+          const float4* row = reinterpret_cast<const float4*>(pl + j1 * RL);
+          float4 v[NP];
+#pragma unroll
+          for (int q = 0; q < NP; ++q) v[q] = row[q];
+          float rx = 0.f, ry = 0.f;
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            rx += wt2[tr][2 * q] * v[q].x;
+            ry += wt2[tr][2 * q] * v[q].y;
+            if (2 * q + 1 < NC) {
+              rx += wt2[tr][2 * q + 1 < NC ? 2 * q + 1 : 0] * v[q].z;
+              ry += wt2[tr][2 * q + 1 < NC ? 2 * q + 1 : 0] * v[q].w;
+            }
+          }
+          sx += wt1[tr][j1] * rx;
+          sy += wt1[tr][j1] * ry;
+        }
+        // x - x is 0 for a finite x only
+        if ((sx - sx) + (sy - sy) != 0.f) {
+          sx = sy = 0.f;
+#pragma unroll
+          for (int j1 = 0; j1 < W; ++j1) {
+            const float2* row = pl + j1 * RL + (odd[tr] ? 1 : 0);
+            float rx = 0.f, ry = 0.f;
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+              const float w0j = wt2[tr][j], w1j = wt2[tr][j + 1];
+              const float w = odd[tr] ? w1j : w0j;
+              rx += w * row[j].x;
+              ry += w * row[j].y;
+            }
+            sx += wt1[tr][j1] * rx;
+            sy += wt1[tr][j1] * ry;
+          }
+        }
+        sx *= w0[tr];
+        sy *= w0[tr];
+      }
+      sx = point_sum(sx);
+      sy = point_sum(sy);
+      if (live[tr] && s == 0) {
+        float2 r = make_float2(a.scale * sx, a.scale * sy);
+        if (a.mode == 1) {
+          r.x = (r.x - y[tr].x) * dens[tr];
+          r.y = (r.y - y[tr].y) * dens[tr];
+          a.out[(int64_t)(t0 + gg) * a.g.M + pb + tr * (NT / 8) + wave * 8 + slot] = r;
+        } else {
+          a.out[kbase[tr] + (t0 + gg) * kstep] = r;
+        }
       }
     }
   }
@@ -2403,6 +2712,37 @@ int launch_interp(const hipnufft_plan_s* p, const float2* grid, int64_t grid_str
   a.mode = mode;
   if (region_lds_bytes(p, 1) > kMaxLdsRegion)
     return set_error(HIPNUFFT_ERR_ARG, "interp tile too large for LDS");
+  // aligned pairs of cells (see k_interp_stream): even last axis and tile,
+  // 16-byte aligned grids
+  const bool pair = p->nf[2] % 2 == 0 && p->tile[2] % 2 == 0 && grid_stride % 2 == 0 &&
+                    reinterpret_cast<uintptr_t>(grid) % 16 == 0;
+  const int pair_rl = (region_extent(p, 2) + ((p->w / 2) & 1) + 1) / 2 * 2;
+  if (p->ndim == 3 && p->interp_group <= 0 && pair && p->w <= kStreamMaxW &&
+      p->max_sub <= kPairPoints && grid_size(p) < ((int64_t)1 << 28)) {
+    const int ps = pair_plane_stride(region_extent(p, 1) * pair_rl);
+    const int64_t rows = (int64_t)region_extent(p, 0) * region_extent(p, 1);
+    set_region_magic(p, &a, kPairNT);
+    if (((int64_t)region_extent(p, 0) * ps + 127) / 128 * 128 <= kPairCells &&
+        rows <= kStreamRows && a.wrap1) {
+      a.lds_row_mag = magic_of(pair_rl);
+      a.lds_plane_mag = magic_of(ps);
+      a.grid_bytes = (int)(grid_size(p) * (int64_t)sizeof(float2));
+      a.sub_mask = p->mask_rows > 0 ? p->sub_mask : nullptr;
+      // transforms per workgroup: all of the set's, fewer when the items
+      // alone give less than two workgroups per CU twice over
+      int Gs = r.ts;
+      while (Gs > 1 && nsub * (int64_t)((r.ts + Gs - 1) / Gs) < 1024) Gs = (Gs + 1) / 2;
+      a.G = Gs;
+      const dim3 grd((unsigned)nsub, (unsigned)((r.ts + Gs - 1) / Gs));
+      StageScope timer(p, kStageInterp);
+      HN_WIDTH_SWITCH(p->w, {
+        if constexpr (WW <= kStreamMaxW)
+          hipLaunchKernelGGL((k_interp_pairs<WW>), grd, dim3(kPairNT), 0, p->stream, a);
+      });
+      HN_LAUNCH_CHECK();
+      return 0;
+    }
+  }
   if (p->ndim >= 2 && p->interp_group <= 0) {
     // every transform of an item in one workgroup (k_interp_stream) when
     // its region, grid and items fit the kernel
@@ -2412,13 +2752,14 @@ int launch_interp(const hipnufft_plan_s* p, const float2* grid, int64_t grid_str
     int64_t cells = 1;
     for (int d = 3 - p->ndim; d < 3; ++d) cells *= region_extent(p, d);
     const int64_t rows = cells / region_extent(p, 2);
-    const int64_t padded = (rows * (region_extent(p, 2) + kStreamPad) + 31) / 32 * 32;
+    const int64_t rl = pair ? pair_rl : region_extent(p, 2);
+    const int64_t seg = pair ? 128 : 32;
+    const int64_t padded = (rows * rl + seg - 1) / seg * seg;
     if (padded <= (d3 ? kStreamCells : kStream2Cells) && rows <= (d3 ? kStreamRows : kStream2Rows) &&
         grid_size(p) < ((int64_t)1 << 28) && p->max_sub <= (NT >= 1024 ? NT / 2 : NT) &&
         p->w <= kStreamMaxW) {
       set_region_magic(p, &a, NT);
-      a.lds_pad = kStreamPad;
-      a.lds_row_mag = magic_of(region_extent(p, 2) + kStreamPad);
+      a.lds_row_mag = magic_of(rl);
       a.grid_bytes = (int)(grid_size(p) * (int64_t)sizeof(float2));
       a.sub_mask = p->mask_rows > 0 ? p->sub_mask : nullptr;
       // transforms per workgroup: all of the set's, fewer when the items
@@ -2426,27 +2767,37 @@ int launch_interp(const hipnufft_plan_s* p, const float2* grid, int64_t grid_str
       // workgroups (two per CU).  2D (eight per CU): at least 16384, dense
       // items then leave no tail (stacked 128^3 slices, 2048 transforms:
       // 0.37 ms less per type 2 than with 4096), but at least 16 transforms
-      // each, over which the point set-up is shared (radial 256^2, 64 coils:
-      // 0.228 ms at 4 transforms, 0.195 at 16)
+      // each, over which the point set-up is shared (1024 stacked planes:
+      // 0.57 ms at 4, 0.49 at 8, 0.46 at 16); below 16 only while the chip
+      // is not full at all (320^2, 32 coils, 684 items: 61 us at 32, 52 at
+      // 16, 46 at 8; 256^2, 8 coils, 361 items: 20 us at 8, 16 at 4)
       int Gs = r.ts;
       if (d3) {
         while (Gs > 1 && nsub * (int64_t)((r.ts + Gs - 1) / Gs) < 1024) Gs = (Gs + 1) / 2;
       } else {
-        while (Gs > 16 && nsub * (int64_t)((r.ts + Gs - 1) / Gs) < 16384) Gs = (Gs + 1) / 2;
+        auto wgs = [&] { return nsub * (int64_t)((r.ts + Gs - 1) / Gs); };
+        while ((Gs > 16 && wgs() < 16384) || (Gs > 4 && wgs() < 2048)) Gs = (Gs + 1) / 2;
       }
       a.G = Gs;
       const dim3 grd((unsigned)nsub, (unsigned)((r.ts + Gs - 1) / Gs));
       StageScope timer(p, kStageInterp);
+#define HN_STREAM(PP)                                                                            \
+  if (d3)                                                                                         \
+    hipLaunchKernelGGL((k_interp_stream<3, WW, kStreamNT, NB, kStreamCells, kStreamRows, PP>), grd, \
+                       dim3(NT), 0, p->stream, a);                                                \
+  else                                                                                            \
+    hipLaunchKernelGGL((k_interp_stream<2, WW, kStream2NT, NB, kStream2Cells, kStream2Rows, PP>), \
+                       grd, dim3(NT), 0, p->stream, a);
       HN_WIDTH_SWITCH(p->w, {
         if constexpr (WW <= kStreamMaxW) {
-          if (d3)
-            hipLaunchKernelGGL((k_interp_stream<3, WW, kStreamNT, NB, kStreamCells, kStreamRows>),
-                               grd, dim3(NT), 0, p->stream, a);
-          else
-            hipLaunchKernelGGL((k_interp_stream<2, WW, kStream2NT, NB, kStream2Cells, kStream2Rows>),
-                               grd, dim3(NT), 0, p->stream, a);
+          if (pair) {
+            HN_STREAM(true)
+          } else {
+            HN_STREAM(false)
+          }
         }
       });
+#undef HN_STREAM
       HN_LAUNCH_CHECK();
       return 0;
     }
