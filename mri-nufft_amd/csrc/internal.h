@@ -45,6 +45,9 @@ inline bool injected_failure(const char* site) {
                              std::string("kernel launch: ") + hipGetErrorString(e_)); \
   } while (0)
 
+constexpr int kMaskWords = 2;       // 64-bit words of a line mask
+constexpr int kMaskTiles = 64 * kMaskWords;
+
 // One FFT axis: length, radix plan, twiddle table, lines per workgroup.
 struct FFTAxis {
   int n = 1;
@@ -155,6 +158,13 @@ struct hipnufft_plan_s {
   uint16_t* sub_mask = nullptr;
   int64_t sub_mask_cap = 0;
   int mask_rows = 0;
+  // support of the points' footprints on the fine grid, in tiles (see
+  // build_line_masks): which tiles along axis 0 a footprint of any set
+  // touches, per (tile of axis 1, tile of axis 2), then which tiles along
+  // axis 1 one touches anywhere, per tile of axis 2; kMaskWords words each.
+  // The rest of the grid is neither written nor read (prune = 0: all of it is).
+  uint64_t* line_mask = nullptr;
+  int prune = 0;
   int32_t* list_pts = nullptr;    // spread lists (sorted-point positions)
   int32_t* list_start = nullptr;  // nsets * nbins + 1
   int64_t nlist = 0;
@@ -231,14 +241,18 @@ struct BlockIdx3 {
   int x, y, z;
 };
 __device__ __forceinline__ BlockIdx3 remapped_block() {
-  const int64_t nx = gridDim.x, ny = gridDim.y;
-  const int64_t n = nx * ny * gridDim.z;
-  const int64_t b = blockIdx.x + nx * (blockIdx.y + ny * (int64_t)blockIdx.z);
-  const int64_t l = xcd_remap(b, n);
+  // 32 bits: 2^31 workgroups would own more data than the memory holds
+  const uint32_t nx = gridDim.x, ny = gridDim.y;
+  const uint32_t n = nx * ny * gridDim.z;
+  const uint32_t b = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
+  const uint32_t l = (uint32_t)xcd_remap(b, n);
+  // (the divisions leave the results in vector registers: back to scalars,
+  // so that addresses formed from them are uniform)
+  const uint32_t yz = __builtin_amdgcn_readfirstlane(l / nx);
   BlockIdx3 r;
-  r.x = (int)(l % nx);
-  r.y = (int)((l / nx) % ny);
-  r.z = (int)(l / (nx * ny));
+  r.x = (int)(l - yz * nx);
+  r.z = __builtin_amdgcn_readfirstlane(yz / ny);
+  r.y = (int)(yz - (uint32_t)r.z * ny);
   return r;
 }
 
