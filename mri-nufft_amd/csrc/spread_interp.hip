@@ -60,6 +60,7 @@ struct SpreadArgs {
   int64_t grid_stride;
   int k0, ts;               // SetRange of the launch
   int G;
+  int out_pairs;            // grid cells may be stored in 16-byte pairs
 };
 
 struct InterpArgs {
@@ -445,47 +446,76 @@ __device__ __forceinline__ uint32_t axis_weights(float* wr, int st, float off, i
   return hit;
 }
 
-// Record of an entry for the matrix-core kernel at sp: touched-block mask,
-// G strengths and, per axis, the weight of every tile cell along it (zero
-// outside the footprint and past the grid end).  A lane's weights for a
-// block then sit at fixed offsets from the record: no header lookup before
-// the reads.  Same weights as the block record, so the same products.
+// Record of an entry for the matrix-core kernel at sp: the blocks that its
+// footprint meets along each axis (bits 0-7: axis 0, 8-15: axis 1 of three,
+// 16-31: the last axis), G strengths and, per axis, the weight of every tile
+// cell along it (zero outside the footprint and past the grid end).  A lane's
+// weights for a block then sit at fixed offsets from the record: no header
+// lookup before the reads.  Same weights as the block record, so the same
+// products.
 __host__ __device__ constexpr int mfma_record_floats(int G, int tiles_sum) {
   return (kBlkHead + 2 * G + tiles_sum + 3) & ~3;
 }
 
+// the header bits of a block: an entry touches it if it has all of them
+template <int D>
+__device__ __forceinline__ uint32_t block_bits(const int* bidx) {
+  return D == 3 ? 1u << bidx[0] | 256u << bidx[1] | 65536u << bidx[2]
+                : 1u << bidx[0] | 65536u << bidx[1];
+}
+
+// One half of an entry's record, each written by a wave of its own: `last`
+// selects the last axis (and in 3D all strengths), the other half the axes
+// before it; in 2D the halves share the strengths.  The kernel evaluations
+// are the longest phase of a round: written by one thread per entry, half of
+// the waves wrote whole records while the other half, and the SIMDs they run
+// on, waited (in every workgroup the same half).  192^3, 16 coils: 3.35 ->
+// 3.17 ms, 1024 stacked 128^2 planes 1.73 -> 1.52, 320^2, 32 coils 0.166 ->
+// 0.145.  (Split over the two lanes of a pair instead, the kernel spilled.)
 template <int D, int G>
-__device__ __forceinline__ void write_mfma_entry(float* sp, const BlkPos& r, const SpreadArgs& a,
-                                                 int t0, int Gv, const int* td, const int* ext,
-                                                 const int* nf, const int* nb, float inv_hw,
-                                                 float beta) {
+__device__ __forceinline__ void write_mfma_half(float* sp, bool last, int p, const SpreadArgs& a,
+                                                int t0, int Gv, const int* org, const int* td,
+                                                const int* ext, const int* nf, float inv_hw,
+                                                float beta) {
+  constexpr int DL = D - 1;
+  constexpr bool A4 = (kBlkHead + 2 * G) % 4 == 0;
+  constexpr int GH0 = D == 3 ? 0 : G / 2;  // strengths [0, GH0) by the first half
   const int W = a.g.w;
-  float2 v[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-    v[g] = g < Gv ? a.in[(int64_t)(t0 + g) * a.in_stride + r.p] : make_float2(0.f, 0.f);
-  uint32_t hit[3] = {1u, 1u, 1u};
   float* wr = sp + kBlkHead + 2 * G;
+  uint16_t* head = reinterpret_cast<uint16_t*>(sp);
+  float2* sv = reinterpret_cast<float2*>(sp + kBlkHead);
+  if (last) {
+    const float off = a.g.off[DL][p];
+    const int st = a.g.cell[DL][p] - org[DL];
+    float2 v[G - GH0];
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
+    for (int g = GH0; g < G; ++g)
+      v[g - GH0] = g < Gv ? a.in[(int64_t)(t0 + g) * a.in_stride + p] : make_float2(0.f, 0.f);
     // blocks of 4 cells along each axis, 16 along the last in 2D
-    hit[d] = axis_weights<(kBlkHead + 2 * G) % 4 == 0>(
-        wr, r.st[d], r.off[d], nf[d], td[d], ext[d], W,
-        D == 2 && d == 1 ? 4 * kBlkE : kBlkE, inv_hw, beta);
-    wr += td[d];
-  }
-  uint32_t mask = 0u;
-  for (int b0 = 0; b0 < nb[0]; ++b0)
-    for (int b1 = 0; b1 < nb[1]; ++b1)
-      for (int b2 = 0; b2 < nb[2]; ++b2)
-        if ((hit[0] >> b0) & (hit[1] >> b1) & (hit[2] >> b2) & 1u)
-          mask |= 1u << ((b0 * nb[1] + b1) * nb[2] + b2);
-  reinterpret_cast<uint32_t*>(sp)[0] = mask;
-  float* sv = sp + kBlkHead;
+    head[1] = (uint16_t)axis_weights<A4>(wr + td[0] + (D == 3 ? td[1] : 0), st, off, nf[DL], td[DL],
+                                         ext[DL], W, D == 2 ? 4 * kBlkE : kBlkE, inv_hw, beta);
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    sv[2 * g] = v[g].x;
-    sv[2 * g + 1] = v[g].y;
+    for (int g = GH0; g < G; ++g) sv[g] = v[g - GH0];
+  } else {
+    const float off0 = a.g.off[0][p];
+    const int st0 = a.g.cell[0][p] - org[0];
+    float off1 = 0.f;
+    int st1 = 0;
+    if constexpr (D == 3) {
+      off1 = a.g.off[1][p];
+      st1 = a.g.cell[1][p] - org[1];
+    }
+    float2 v[GH0 > 0 ? GH0 : 1];
+#pragma unroll
+    for (int g = 0; g < GH0; ++g)
+      v[g] = g < Gv ? a.in[(int64_t)(t0 + g) * a.in_stride + p] : make_float2(0.f, 0.f);
+    uint32_t hit = axis_weights<A4>(wr, st0, off0, nf[0], td[0], ext[0], W, kBlkE, inv_hw, beta);
+    if constexpr (D == 3)
+      hit |= axis_weights<A4>(wr + td[0], st1, off1, nf[1], td[1], ext[1], W, kBlkE, inv_hw, beta)
+             << 8;
+    head[0] = (uint16_t)hit;
+#pragma unroll
+    for (int g = 0; g < GH0; ++g) sv[g] = v[g];
   }
 }
 
@@ -692,7 +722,7 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
     bool live = b < nblk;
 #pragma unroll
     for (int d = 0; d < D; ++d) live = live && bidx[bi][d] * (d == D - 1 ? BL : kBlkE) < ext[d];
-    bbit[bi] = live ? 1u << b : 0u;
+    bbit[bi] = live ? block_bits<D>(bidx[bi]) : 0u;
   }
 
   f32x4 acc[BPW][kBlkE][GH];
@@ -703,10 +733,13 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
 #pragma unroll
       for (int h = 0; h < GH; ++h) acc[bi][s][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  constexpr int CHUNK = kBlkChunk * NWAVE / 4;  // staged entries per round (a multiple of 64)
+  constexpr int CHUNK = kBlkChunk * NWAVE / 4;  // staged entries per round: 64 per wave pair
+  static_assert(2 * CHUNK == 64 * NWAVE, "two threads per staged entry");
   const int e0 = a.it_begin[item];
   const int e1 = min(e0 + a.smax, a.list_start[key + 1]);
-  const int q = (int)threadIdx.x;
+  // thread -> entry of the round, half of its record (uniform in a wave)
+  const int q = (int)threadIdx.x & (CHUNK - 1);
+  const bool last = wave >= NWAVE / 2;
   // per block of the wave, the record offsets (floats from smem) of the
   // staged entries that touch it, in list order; a zero record after the
   // staged ones pads the last group of four
@@ -732,11 +765,8 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
   for (int eb = e0; eb < e1; eb += CHUNK) {
     const int n = min(CHUNK, e1 - eb);
     const int pcur = pnext;
-    if (q < n) {
-      BlkPos r;
-      load_blk_pos<D>(a, pcur, org, r);
-      write_mfma_entry<D, G>(smem + q * PW, r, a, t0, Gv, td, ext, nf, nb, inv_hw, beta);
-    }
+    if (q < n)
+      write_mfma_half<D, G>(smem + q * PW, last, pcur, a, t0, Gv, org, td, ext, nf, inv_hw, beta);
     // in flight during this round's lists and products
     if (q < min(CHUNK, e1 - eb - CHUNK)) pnext = a.list_pts[eb + CHUNK + q];
     __syncthreads();
@@ -750,7 +780,7 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
           const int qi = base + lane;
           const uint32_t hm =
               qi < n ? reinterpret_cast<const uint32_t*>(smem + qi * PW)[0] : 0u;
-          const bool hit = (hm & bbit[bi]) != 0u;
+          const bool hit = (hm & bbit[bi]) == bbit[bi];
           const uint64_t bal = __ballot(hit);
           if (hit) lst[cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] =
@@ -792,55 +822,58 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
     __syncthreads();
   }
 
-  // register r of lane l holds value l % 16 (transform 8 h + (l % 16) / 2,
+  // Register r of lane l holds value l % 16 (transform 8 h + (l % 16) / 2,
   // re / im by parity) of cell (slice, l / 16, r); lanes 2g and 2g + 1 swap
-  // halves so that each writes two whole complex cells
+  // halves (by DPP: through LDS, these exchanges took longer than the stores)
+  // so that each stores two whole complex cells at once, at a lane pointer
+  // plus one uniform offset per slice.  (Sorted through LDS into whole rows
+  // first, the write-out was slower: 3.87 against 3.35 ms at 192^3, 16 coils;
+  // this form took that kernel from 3.17 to 2.87.)
   const int TC = td[0] * td[1] * td[2];
   const bool odd = lane & 1;
   const int ry = lane >> 4;
+  const bool part = slot >= 0;  // partial tile of a dense tile: summed by k_spread_reduce
+  const int64_t s1 = part ? td[D - 1] : nf[D - 1];              // cells between rows
+  const int64_t s0 = part ? (D == 3 ? td[1] * s1 : s1) : (D == 3 ? nf[1] * s1 : s1);
+  const int64_t tstride = part ? (int64_t)TC : a.grid_stride;
+  float2* base = part ? a.part + ((int64_t)slot * a.ntrans + tb + t0) * TC
+                      : a.grid + (int64_t)(tb + t0) * a.grid_stride + org[0] * s0 +
+                            (D == 3 ? org[1] * s1 + org[2] : org[1]);
+  const int lz = (D == 3 ? 0 : 4 * ry) + (odd ? 2 : 0);  // the lane's first cell along the rows
+  float2* lp = base + ((lane & 15) >> 1) * tstride + (D == 3 ? ry * s1 : 0) + lz;
+  const bool pairs = part || a.out_pairs;
 #pragma unroll
   for (int bi = 0; bi < BPW; ++bi) {
     if (!bbit[bi]) continue;
+    const int zb = D == 3 ? bidx[bi][2] * kBlkE : bidx[bi][1] * BL;  // uniform
+    const int zl = ext[D - 1] - zb - lz;  // cells from the lane's first to the end
+    const bool rok = zl > 0 && (D == 2 || bidx[bi][1] * kBlkE + ry < ext[1]);
+    const int64_t bo = (D == 3 ? bidx[bi][1] * kBlkE * s1 : 0) + zb;
 #pragma unroll
     for (int sx = 0; sx < kBlkE; ++sx) {
+      const int c0 = bidx[bi][0] * kBlkE + sx;  // uniform
 #pragma unroll
       for (int hh = 0; hh < GH; ++hh) {
-        float2 out[2];
+        f32x4 o;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           // even lane keeps cells r = 0, 1, odd lane cells r = 2, 3
           const float mine = odd ? acc[bi][sx][hh][2 + h] : acc[bi][sx][hh][h];
           const float give = odd ? acc[bi][sx][hh][h] : acc[bi][sx][hh][2 + h];
-          const float other = __shfl_xor(give, 1);
-          out[h] = odd ? make_float2(other, mine) : make_float2(mine, other);
+          const float other = __builtin_bit_cast(
+              float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0xB1, 0xf, 0xf,
+                                                 true));  // of lane ^ 1
+          o[2 * h] = odd ? other : mine;
+          o[2 * h + 1] = odd ? mine : other;
         }
-        const int g = 8 * hh + ((lane & 15) >> 1);
-        if (g >= Gv) continue;
-        const int c0 = bidx[bi][0] * kBlkE + sx;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if constexpr (D == 3) {
-            const int c1 = bidx[bi][1] * kBlkE + ry;
-            const int c2 = bidx[bi][2] * kBlkE + (odd ? 2 : 0) + h;
-            if (c0 >= ext[0] || c1 >= ext[1] || c2 >= ext[2]) continue;
-            if (slot >= 0) {
-              const int r = (c0 * td[1] + c1) * td[2] + c2;
-              a.part[((int64_t)slot * a.ntrans + tb + t0 + g) * TC + r] = out[h];
-            } else {
-              const int64_t gi =
-                  ((int64_t)(org[0] + c0) * nf[1] + org[1] + c1) * nf[2] + org[2] + c2;
-              a.grid[(int64_t)(tb + t0 + g) * a.grid_stride + gi] = out[h];
-            }
-          } else {  // row cell 4 ry + r of the block's 16 along the last axis
-            const int c1 = bidx[bi][1] * BL + 4 * ry + (odd ? 2 : 0) + h;
-            if (c0 >= ext[0] || c1 >= ext[1]) continue;
-            if (slot >= 0) {
-              const int r = c0 * td[1] + c1;
-              a.part[((int64_t)slot * a.ntrans + tb + t0 + g) * TC + r] = out[h];
-            } else {
-              const int64_t gi = (int64_t)(org[0] + c0) * nf[1] + org[1] + c1;
-              a.grid[(int64_t)(tb + t0 + g) * a.grid_stride + gi] = out[h];
-            }
+        if (c0 >= ext[0]) continue;  // uniform
+        if (rok && 8 * hh + ((lane & 15) >> 1) < Gv) {
+          float2* dst = lp + 8 * hh * tstride + (c0 * s0 + bo);
+          if (pairs) {
+            *reinterpret_cast<f32x4*>(dst) = o;
+          } else {  // odd grid rows (spread / interp only)
+            dst[0] = make_float2(o[0], o[1]);
+            if (zl > 1) dst[1] = make_float2(o[2], o[3]);
           }
         }
       }
@@ -2469,6 +2502,8 @@ int launch_spread_sorted(const hipnufft_plan_s* p, const float2* in, SetRange r,
   a.grid_stride = grid_stride;
   a.k0 = r.k0;
   a.ts = r.ts;
+  a.out_pairs = p->nf[2] % 2 == 0 && grid_stride % 2 == 0 &&
+                reinterpret_cast<uintptr_t>(grid) % 16 == 0;
   a.item0 = (int)p->item_of_set[r.k0];
   a.dn0 = (int)p->dense_of_set[r.k0];
   const int64_t nitems = p->item_of_set[r.k1] - p->item_of_set[r.k0];
