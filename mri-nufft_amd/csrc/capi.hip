@@ -157,6 +157,7 @@ int make_axis(int64_t n, FFTAxis* ax, size_t* bytes, bool allow_direct = false,
   // a remaining factor 2 pairs with a 3 into one radix-6 pass (one LDS round
   // trip fewer): 384 = 8 * 8 * 6
   if (m % 6 == 0) { ax->rad[ax->nrad++] = 6; m /= 6; }
+  if (m % 10 == 0) { ax->rad[ax->nrad++] = 10; m /= 10; }  // likewise with a 5: 640 = 8 * 8 * 10
   if (m % 2 == 0) { ax->rad[ax->nrad++] = 2; m /= 2; }
   while (m % 3 == 0 && ax->nrad < kMaxRadices) { ax->rad[ax->nrad++] = 3; m /= 3; }
   while (m % 5 == 0 && ax->nrad < kMaxRadices) { ax->rad[ax->nrad++] = 5; m /= 5; }

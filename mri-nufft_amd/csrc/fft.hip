@@ -126,6 +126,26 @@ __device__ __forceinline__ void dft6(float2* v) {
   v[5] = csub(a[2], b[2]);
 }
 
+// 10 = 2 x 5 by the same mapping: inputs (5 n1 + 2 n2) mod 10, two 5-point
+// DFTs over n2, 2-point DFTs over n1, outputs at (5 k1 + 6 k2) mod 10
+template <int S>
+__device__ __forceinline__ void dft10(float2* v) {
+  float2 a[5] = {v[0], v[2], v[4], v[6], v[8]};
+  float2 b[5] = {v[5], v[7], v[9], v[1], v[3]};
+  dft5<S>(a);
+  dft5<S>(b);
+  v[0] = cadd(a[0], b[0]);
+  v[5] = csub(a[0], b[0]);
+  v[6] = cadd(a[1], b[1]);
+  v[1] = csub(a[1], b[1]);
+  v[2] = cadd(a[2], b[2]);
+  v[7] = csub(a[2], b[2]);
+  v[8] = cadd(a[3], b[3]);
+  v[3] = csub(a[3], b[3]);
+  v[4] = cadd(a[4], b[4]);
+  v[9] = csub(a[4], b[4]);
+}
+
 template <int R, int S>
 __device__ __forceinline__ void dftR(float2* v) {
   if constexpr (R == 2) dft2<S>(v);
@@ -134,6 +154,7 @@ __device__ __forceinline__ void dftR(float2* v) {
   if constexpr (R == 5) dft5<S>(v);
   if constexpr (R == 6) dft6<S>(v);
   if constexpr (R == 8) dft8<S>(v);
+  if constexpr (R == 10) dft10<S>(v);
 }
 
 // One Stockham radix-R pass over L interleaved lines of length n held in LDS
@@ -243,7 +264,7 @@ __device__ __forceinline__ void stockham_pass_ct(float2* buf, const float2* tw) 
 }
 
 // The p-th radix of the plan of an n-point line: 8s, then at most one each of
-// 4, 6 and 2, then 3s and 5s (0 past the end) -- the rule of the host's axis
+// 4, 6, 10 and 2, then 3s and 5s (0 past the end) -- the rule of the host's axis
 // set-up, so that a compile-time plan can be checked against the runtime one
 __host__ __device__ constexpr int plan_radix(int n, int p) {
   int rad[16] = {};
@@ -251,6 +272,7 @@ __host__ __device__ constexpr int plan_radix(int n, int p) {
   while (m % 8 == 0 && k < 16) { rad[k++] = 8; m /= 8; }
   if (m % 4 == 0) { rad[k++] = 4; m /= 4; }
   if (m % 6 == 0) { rad[k++] = 6; m /= 6; }
+  if (m % 10 == 0) { rad[k++] = 10; m /= 10; }
   if (m % 2 == 0) { rad[k++] = 2; m /= 2; }
   while (m % 3 == 0 && k < 16) { rad[k++] = 3; m /= 3; }
   while (m % 5 == 0 && k < 16) { rad[k++] = 5; m /= 5; }
@@ -292,6 +314,7 @@ __device__ void fft_lines(float2* buf, const float2* twl, const FFTAxis& ax, int
       case 4: stockham_pass<4, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
       case 5: stockham_pass<5, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
       case 6: stockham_pass<6, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
+      case 10: stockham_pass<10, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
       default: stockham_pass<8, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
     }
     Ns *= R;
@@ -969,28 +992,39 @@ int lg2(int x) {
   return l;
 }
 
-size_t fft_lds(const FFTAxis& ax) { return sizeof(float2) * (size_t)ax.n * (ax.L + 2); }
+size_t fft_lds(const FFTAxis& ax, int L) { return sizeof(float2) * (size_t)ax.n * (L + 2); }
+size_t fft_lds(const FFTAxis& ax) { return fft_lds(ax, ax.L); }
 
-// the axis has n points on L lines and the runtime radix plan is the
-// compile-time one of fft_lines_ct
-bool fixed_plan(const FFTAxis& ax, int n, int L) {
-  if (ax.n != n || ax.L != L || ax.direct) return false;
+// the axis has n points and its runtime radix plan is the compile-time one
+// of fft_lines_ct
+bool fixed_plan(const FFTAxis& ax, int n) {
+  if (ax.n != n || ax.direct) return false;
   int p = 0;
   for (; p < ax.nrad; ++p)
     if (ax.rad[p] != plan_radix(n, p)) return false;
   return plan_radix(n, p) == 0;
 }
 
-// complex elements per thread for the L lines of n elements of an axis:
-// the smallest of 8, 12, 16 with n * L <= EPT * nt (fewer registers,
-// more resident waves for the shorter lines)
-int ept_of(const FFTAxis& ax, int nt = kThreads) {
-  const int need = (ax.n * ax.L + nt - 1) / nt;
-  return need <= 8 ? 8 : need <= 12 ? 12 : 16;
+// complex elements per thread for L lines of n elements: the smallest of 4,
+// 8, 12, 16 with n * L <= EPT * nt (fewer registers, more resident waves for
+// the shorter lines)
+int ept_of(int n, int L, int nt = kThreads) {
+  const int need = (n * L + nt - 1) / nt;
+  return need <= 4 ? 4 : need <= 8 ? 8 : need <= 12 ? 12 : 16;
+}
+
+// Lines per workgroup of a pass over `lines` lines: the axis's L, or a
+// quarter of it where that leaves CUs without any workgroup.  A single 2D
+// image has a few dozen workgroups of L lines, whose threads then walk 12 to
+// 16 elements each with most of the chip idle (256^2, one image: the four
+// passes 33.5 -> 21.9 us).  min_l: fewer lines are not allowed (line masks).
+int lines_of(const FFTAxis& ax, int64_t lines, int min_l = 1) {
+  return ax.L >= 4 && ax.L / 4 >= min_l && lines < 256 * (int64_t)ax.L ? ax.L / 4 : ax.L;
 }
 
 #define HN_EPT_SWITCH(ept, ...)             \
   switch (ept) {                            \
+    case 4: { constexpr int EE = 4; __VA_ARGS__ } break;   \
     case 8: { constexpr int EE = 8; __VA_ARGS__ } break;   \
     case 12: { constexpr int EE = 12; __VA_ARGS__ } break; \
     default: { constexpr int EE = 16; __VA_ARGS__ } break; \
@@ -1033,7 +1067,6 @@ int strided(const hipnufft_plan_s* p, int axis, int T, int in_M, int out_M, int 
   a.in_M = in_M;
   a.out_M = out_M;
   a.ax = ax;
-  a.lgL = lg2(ax.L);
   if (axis == 1) {
     a.lstride = p->nf[2];
     a.ostride = p->nf[1] * p->nf[2];
@@ -1057,29 +1090,40 @@ int strided(const hipnufft_plan_s* p, int axis, int T, int in_M, int out_M, int 
     a.ctile_sh = lg2(p->tile[2]);
     a.zero_empty = axis == 1 && out_M != 0;
   }
-  const dim3 grd((unsigned)((a.nx + ax.L - 1) / ax.L), (unsigned)a.nouter, (unsigned)T);
+  const int L = lines_of(ax, (int64_t)a.nx * a.nouter * T, a.lmask ? 64 / p->tile[axis] : 1);
+  a.lgL = lg2(L);
+  const dim3 grd((unsigned)((a.nx + L - 1) / L), (unsigned)a.nouter, (unsigned)T);
   StageScope timer(p, stage);
-  const size_t lds = fft_lds(ax);
+  const size_t lds = fft_lds(ax, L);
   // strided axes may hold up to 2 * kMaxElemsFFT elements (16 lines of up to
   // 512): those run 512-thread workgroups
-// compile-time plans: (points, log2 lines, threads, elements per thread)
-#define HN_STRIDED_FIXED(NN, LG, NTT, EPTT)                                            \
-  if (fixed_plan(ax, NN, 1 << LG)) {                                                     \
+// compile-time plans: points, log2 lines, threads, elements per thread
+#define HN_STRIDED_FIXED(NN, LG, NTT, EPTT)                                   \
+  if (L == 1 << LG && fixed_plan(ax, NN)) {                                     \
     launch_strided<EPTT, NTT, NN, LG>(K != nullptr, sign, grd, lds, p->stream, a); \
-    HN_LAUNCH_CHECK();                                                                   \
-    return 0;                                                                            \
+    HN_LAUNCH_CHECK();                                                          \
+    return 0;                                                                   \
   }
   HN_STRIDED_FIXED(384, 4, 2 * kThreads, 12)
+  HN_STRIDED_FIXED(384, 2, 2 * kThreads, 3)
   HN_STRIDED_FIXED(256, 4, kThreads, 16)
+  HN_STRIDED_FIXED(256, 2, kThreads, 4)
   HN_STRIDED_FIXED(512, 3, kThreads, 16)
+  HN_STRIDED_FIXED(512, 1, kThreads, 4)
   HN_STRIDED_FIXED(768, 3, 2 * kThreads, 12)
+  HN_STRIDED_FIXED(768, 1, 2 * kThreads, 3)
+  HN_STRIDED_FIXED(640, 3, 2 * kThreads, 10)
+  HN_STRIDED_FIXED(640, 1, 2 * kThreads, 3)
+  HN_STRIDED_FIXED(320, 4, 2 * kThreads, 10)
+  HN_STRIDED_FIXED(192, 4, kThreads, 12)
+  HN_STRIDED_FIXED(128, 4, kThreads, 8)
 #undef HN_STRIDED_FIXED
-  if (ax.n * ax.L > kMaxElemsFFT) {
-    HN_EPT_SWITCH(ept_of(ax, 2 * kThreads), {
+  if (ax.n * L > kMaxElemsFFT) {
+    HN_EPT_SWITCH(ept_of(ax.n, L, 2 * kThreads), {
       launch_strided<EE, 2 * kThreads>(K != nullptr, sign, grd, lds, p->stream, a);
     });
   } else {
-    HN_EPT_SWITCH(ept_of(ax), {
+    HN_EPT_SWITCH(ept_of(ax.n, L), {
       launch_strided<EE, kThreads>(K != nullptr, sign, grd, lds, p->stream, a);
     });
   }
@@ -1133,6 +1177,30 @@ int mul_spectrum(const hipnufft_plan_s* p, const float2* K, int T) {
 
 namespace {
 
+// the row kernels with compile-time plans (points, log2 lines, elements per
+// thread), else the runtime plan (640 points, of 320^2 with 32 coils:
+// forward rows 37 -> 27 us, adjoint rows 70 -> 41, each column pass 58 -> 36)
+#define HN_ROWS_FIXED(NN, LG, EPTT)         \
+  if (L == 1 << LG && fixed_plan(ax, NN)) { \
+    HN_ROWS(EPTT, NN, LG);                  \
+  } else
+#define HN_ROWS_SWITCH                                                    \
+  HN_ROWS_FIXED(384, 3, 12)                                               \
+  HN_ROWS_FIXED(384, 1, 3)                                                \
+  HN_ROWS_FIXED(256, 4, 16)                                               \
+  HN_ROWS_FIXED(256, 2, 4)                                                \
+  HN_ROWS_FIXED(512, 3, 16)                                               \
+  HN_ROWS_FIXED(512, 1, 4)                                                \
+  HN_ROWS_FIXED(768, 2, 12)                                               \
+  HN_ROWS_FIXED(768, 0, 3)                                                \
+  HN_ROWS_FIXED(640, 2, 10)                                               \
+  HN_ROWS_FIXED(640, 0, 3)                                                \
+  HN_ROWS_FIXED(320, 3, 10)                                               \
+  HN_ROWS_FIXED(192, 4, 12)                                               \
+  HN_ROWS_FIXED(128, 4, 8) {                                              \
+    HN_EPT_SWITCH(ept_of(ax.n, L), { HN_ROWS(EE); });                     \
+  }
+
 int rows_fwd(const hipnufft_plan_s* p, const float2* img, const float2* smaps, int C, int t0, int T,
              float scale, int sign, int conj_smaps, int smaps_all, const float2* cmap = nullptr,
              int nmaps = 1) {
@@ -1148,42 +1216,21 @@ int rows_fwd(const hipnufft_plan_s* p, const float2* img, const float2* smaps, i
   a.T = T;
   a.scale = scale;
   const int rows = a.M0 * a.M1;
-  const int L = p->fft[2].L;
+  const FFTAxis& ax = p->fft[2];
+  const int L = lines_of(ax, (int64_t)rows * T);
+  a.lgL = lg2(L);
   const dim3 grd((unsigned)((rows + L - 1) / L), (unsigned)T);
-  const size_t lds = fft_lds(p->fft[2]);
-  {
-    StageScope timer(p, kStageRowsFwd);
-    const FFTAxis& ax = p->fft[2];
-    if (fixed_plan(ax, 384, 8)) {
-      if (sign < 0)
-        hipLaunchKernelGGL((k_rows_fwd<-1, 12, 384, 3>), grd, dim3(kThreads), lds, p->stream, a);
-      else
-        hipLaunchKernelGGL((k_rows_fwd<1, 12, 384, 3>), grd, dim3(kThreads), lds, p->stream, a);
-    } else if (fixed_plan(ax, 256, 16)) {
-      if (sign < 0)
-        hipLaunchKernelGGL((k_rows_fwd<-1, 16, 256, 4>), grd, dim3(kThreads), lds, p->stream, a);
-      else
-        hipLaunchKernelGGL((k_rows_fwd<1, 16, 256, 4>), grd, dim3(kThreads), lds, p->stream, a);
-    } else if (fixed_plan(ax, 512, 8)) {
-      if (sign < 0)
-        hipLaunchKernelGGL((k_rows_fwd<-1, 16, 512, 3>), grd, dim3(kThreads), lds, p->stream, a);
-      else
-        hipLaunchKernelGGL((k_rows_fwd<1, 16, 512, 3>), grd, dim3(kThreads), lds, p->stream, a);
-    } else if (fixed_plan(ax, 768, 4)) {
-      if (sign < 0)
-        hipLaunchKernelGGL((k_rows_fwd<-1, 12, 768, 2>), grd, dim3(kThreads), lds, p->stream, a);
-      else
-        hipLaunchKernelGGL((k_rows_fwd<1, 12, 768, 2>), grd, dim3(kThreads), lds, p->stream, a);
-    } else {
-      HN_EPT_SWITCH(ept_of(p->fft[2]), {
-        if (sign < 0)
-          hipLaunchKernelGGL((k_rows_fwd<-1, EE>), grd, dim3(kThreads), lds, p->stream, a);
-        else
-          hipLaunchKernelGGL((k_rows_fwd<1, EE>), grd, dim3(kThreads), lds, p->stream, a);
-      });
-    }
-    HN_LAUNCH_CHECK();
-  }
+  const size_t lds = fft_lds(ax, L);
+  StageScope timer(p, kStageRowsFwd);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grd, dim3(kThreads), lds, p->stream, a);
+  };
+#define HN_ROWS(...)                            \
+  if (sign < 0) go(k_rows_fwd<-1, __VA_ARGS__>); \
+  else go(k_rows_fwd<1, __VA_ARGS__>)
+  HN_ROWS_SWITCH
+#undef HN_ROWS
+  HN_LAUNCH_CHECK();
   return 0;
 }
 
@@ -1200,9 +1247,11 @@ int rows_adj(const hipnufft_plan_s* p, float2* img, const float2* smaps, int C, 
   a.T = T;
   a.scale = scale;
   const int rows = a.M0 * a.M1;
-  const int L = p->fft[2].L;
+  const FFTAxis& ax = p->fft[2];
   const int per_img = (smaps ? C : 1) * nmaps;
   const int nimg = (t0 + T - 1) / per_img - t0 / per_img + 1;
+  const int L = lines_of(ax, (int64_t)rows * std::min(T, per_img * nimg));
+  a.lgL = lg2(L);
   // transforms of an image side by side while the rows alone give fewer than
   // two workgroups per CU (each then walks fewer coils)
   while ((1 << a.lgQ) < L && (1 << a.lgQ) < std::min(per_img, T) &&
@@ -1210,37 +1259,16 @@ int rows_adj(const hipnufft_plan_s* p, float2* img, const float2* smaps, int C, 
     ++a.lgQ;
   const int R = L >> a.lgQ;
   const dim3 grd((unsigned)((rows + R - 1) / R), (unsigned)nimg);
-  const size_t lds = rows_adj_lds(p->fft[2], a.M2);
+  const size_t lds = fft_lds(ax, L) + sizeof(float2) * (size_t)a.M2 * L;
   StageScope timer(p, kStageRowsAdj);
-  const FFTAxis& ax = p->fft[2];
-  if (fixed_plan(ax, 384, 8)) {
-    if (sign < 0)
-      hipLaunchKernelGGL((k_rows_adj<-1, 12, 384, 3>), grd, dim3(kThreads), lds, p->stream, a);
-    else
-      hipLaunchKernelGGL((k_rows_adj<1, 12, 384, 3>), grd, dim3(kThreads), lds, p->stream, a);
-  } else if (fixed_plan(ax, 256, 16)) {
-    if (sign < 0)
-      hipLaunchKernelGGL((k_rows_adj<-1, 16, 256, 4>), grd, dim3(kThreads), lds, p->stream, a);
-    else
-      hipLaunchKernelGGL((k_rows_adj<1, 16, 256, 4>), grd, dim3(kThreads), lds, p->stream, a);
-  } else if (fixed_plan(ax, 512, 8)) {
-    if (sign < 0)
-      hipLaunchKernelGGL((k_rows_adj<-1, 16, 512, 3>), grd, dim3(kThreads), lds, p->stream, a);
-    else
-      hipLaunchKernelGGL((k_rows_adj<1, 16, 512, 3>), grd, dim3(kThreads), lds, p->stream, a);
-  } else if (fixed_plan(ax, 768, 4)) {
-    if (sign < 0)
-      hipLaunchKernelGGL((k_rows_adj<-1, 12, 768, 2>), grd, dim3(kThreads), lds, p->stream, a);
-    else
-      hipLaunchKernelGGL((k_rows_adj<1, 12, 768, 2>), grd, dim3(kThreads), lds, p->stream, a);
-  } else {
-    HN_EPT_SWITCH(ept_of(p->fft[2]), {
-      if (sign < 0)
-        hipLaunchKernelGGL((k_rows_adj<-1, EE>), grd, dim3(kThreads), lds, p->stream, a);
-      else
-        hipLaunchKernelGGL((k_rows_adj<1, EE>), grd, dim3(kThreads), lds, p->stream, a);
-    });
-  }
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grd, dim3(kThreads), lds, p->stream, a);
+  };
+#define HN_ROWS(...)                            \
+  if (sign < 0) go(k_rows_adj<-1, __VA_ARGS__>); \
+  else go(k_rows_adj<1, __VA_ARGS__>)
+  HN_ROWS_SWITCH
+#undef HN_ROWS
   HN_LAUNCH_CHECK();
   return 0;
 }
@@ -1312,7 +1340,7 @@ int stack_fwd(const StackGeom& g, const float2* img, const float2* smaps, int C,
   a.ax = g.ax;
   a.lgL = lg2(g.ax.L);
   const dim3 grd((unsigned)((g.rows + g.ax.L - 1) / g.ax.L), (unsigned)T);
-  HN_EPT_SWITCH(ept_of(g.ax), {
+  HN_EPT_SWITCH(ept_of(g.ax.n, g.ax.L), {
     hipLaunchKernelGGL((k_stack_fwd<EE>), grd, dim3(kThreads), fft_lds(g.ax), s, a);
   });
   HN_LAUNCH_CHECK();
@@ -1337,7 +1365,7 @@ int stack_adj(const StackGeom& g, const float2* planes, const float2* smaps, int
   a.lgL = lg2(g.ax.L);
   const int nimg = smaps ? ((t0 + T - 1) / C - t0 / C + 1) : T;
   const dim3 grd((unsigned)((g.rows + g.ax.L - 1) / g.ax.L), (unsigned)nimg);
-  HN_EPT_SWITCH(ept_of(g.ax), {
+  HN_EPT_SWITCH(ept_of(g.ax.n, g.ax.L), {
     hipLaunchKernelGGL((k_stack_adj<EE>), grd, dim3(kThreads), fft_lds(g.ax), s, a);
   });
   HN_LAUNCH_CHECK();
