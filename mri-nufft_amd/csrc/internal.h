@@ -375,9 +375,7 @@ int rss_normalize(float2* maps, int C, int64_t N, float eps, hipStream_t s);
 int blur_magnitude(float2* maps, int C, int ndim, const int64_t* shape, const double* sigma,
                    double truncate, float* work, hipStream_t s);
 
-// Exclusive scan of n int32 (device), result in out (may alias in), total in
-// *total (host, synchronises the stream) if total != nullptr.
-int scan_exclusive(const int32_t* in, int32_t* out, int64_t n,
-                   hipStream_t s, int64_t* total);
+// Exclusive scan of n int32 (device), result in out (may alias in).
+int scan_exclusive(const int32_t* in, int32_t* out, int64_t n, hipStream_t s);
 
 }  // namespace hn
