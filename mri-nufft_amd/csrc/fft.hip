@@ -477,13 +477,17 @@ __global__ __launch_bounds__(kThreads) void k_rows_fwd(RowsArgs a) {
 // lgQ = 0 against the rule of rows_adj(): 256^2, 8 coils 47.6 -> 10.3 us,
 // 16 coils 89 -> 17; 320^2, 32 coils 233 -> 71; 192^2, 12 frames of 8 coils
 // 43 -> 29.
-template <int S, int EPT, int FIX = 0, int FLGL = 0>
+// SIDE: lgQ > 0 (a walk one by one keeps its transform in scalar registers:
+// 1024 stacked planes, one transform each, 120 us against 155 without the
+// distinction).
+template <int S, int EPT, bool SIDE, int FIX = 0, int FLGL = 0>
 __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   extern __shared__ float2 buf[];
+  const int lgQ = SIDE ? a.lgQ : 0;
   // FIX > 0: FIX-point rows, 2^FLGL per workgroup, passes fixed at compile time
   if constexpr (FIX > 0) a.lgL = FLGL;
   const int L = 1 << a.lgL, LP = L + 1;
-  const int lgR = a.lgL - a.lgQ, R = 1 << lgR, Q = 1 << a.lgQ;
+  const int lgR = a.lgL - lgQ, R = 1 << lgR, Q = 1 << lgQ;
   const float2* twl = stage_twiddles(buf, a.ax, LP);
   const int rows = a.M0 * a.M1;
   const BlockIdx3 bi = remapped_block();
@@ -502,8 +506,8 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   // across the coil loop
   const int TPL = kThreads >> a.lgL;  // threads per line (n <= TPL * EPT)
   const int l = threadIdx.x / TPL, x0 = threadIdx.x - l * TPL;
-  const int q = l & (Q - 1);
-  const int r = r0 + (l >> a.lgQ);
+  const int q = SIDE ? l & (Q - 1) : 0;
+  const int r = r0 + (l >> lgQ);
   const bool rok = r < rows;
   int64_t grow = 0;
   if (rok) {
@@ -516,8 +520,8 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   float2* accl = acc0 + (size_t)l * a.M2;
 
   for (int tg = tb; tg < te; tg += Q) {
-    const int tt = min(tg + q, te - 1);
-    const bool tok = rok && tg + q < te;
+    const int tt = SIDE ? min(tg + q, te - 1) : tg;
+    const bool tok = rok && (!SIDE || tg + q < te);
     const float2* g = a.grid + (int64_t)(tt - a.t0) * a.gstride + grow;
     {
       float2 v[EPT];
@@ -586,7 +590,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
   if (rr >= rows) return;
   const int i0 = rr / a.M1, i1 = rr - i0 * a.M1;
   const float rs = a.dec0[i0] * a.dec1[i1] * a.scale;
-  const float2* accr = acc0 + (size_t)(ro << a.lgQ) * a.M2;
+  const float2* accr = acc0 + (size_t)(ro << lgQ) * a.M2;
   float2* dst = a.img_out + (int64_t)out_img * N + (int64_t)rr * a.M2;
   for (int x = x1; x < a.M2; x += TPR) {
     float2 v = accr[x];
@@ -1264,9 +1268,11 @@ int rows_adj(const hipnufft_plan_s* p, float2* img, const float2* smaps, int C, 
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grd, dim3(kThreads), lds, p->stream, a);
   };
-#define HN_ROWS(...)                            \
-  if (sign < 0) go(k_rows_adj<-1, __VA_ARGS__>); \
-  else go(k_rows_adj<1, __VA_ARGS__>)
+#define HN_ROWS(EPTT, ...)                                                  \
+  if (sign < 0 && a.lgQ) go(k_rows_adj<-1, EPTT, true, ##__VA_ARGS__>);       \
+  else if (sign < 0) go(k_rows_adj<-1, EPTT, false, ##__VA_ARGS__>);          \
+  else if (a.lgQ) go(k_rows_adj<1, EPTT, true, ##__VA_ARGS__>);               \
+  else go(k_rows_adj<1, EPTT, false, ##__VA_ARGS__>)
   HN_ROWS_SWITCH
 #undef HN_ROWS
   HN_LAUNCH_CHECK();
