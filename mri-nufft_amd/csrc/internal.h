@@ -151,7 +151,7 @@ struct hipnufft_plan_s {
   int32_t* pt_idx = nullptr;
   int32_t* bin_start = nullptr;   // nsets * nbins + 1
   int32_t* sub_tile = nullptr;    // interp work items
-  int32_t* sub_begin = nullptr;
+  int32_t* sub_begin = nullptr;   // nsub + 1: the last is the number of points
   int64_t nsub = 0;
   // per interp work item, per row of its staged region: the 16-cell chunks
   // along the last axis its points read (2D / 3D; mask_rows = 0: none)
