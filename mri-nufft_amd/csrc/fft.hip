@@ -475,7 +475,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_fwd(RowsArgs a) {
 // coil's loads, FFT and maps after the other -- so the coils go side by side
 // and their sums meet in LDS at the end, in coil order.  Measured with
 // lgQ = 0 against the rule of rows_adj(): 256^2, 8 coils 47.6 -> 10.3 us,
-// 16 coils 89 -> 17; 320^2, 32 coils 233 -> 71; 192^2, 12 frames of 8 coils
+// 16 coils 89 -> 17; 320^2, 32 coils 233 -> 71 (before its fixed plan); 192^2, 12 frames of 8 coils
 // 43 -> 29.
 // SIDE: lgQ > 0 (a walk one by one keeps its transform in scalar registers:
 // 1024 stacked planes, one transform each, 120 us against 155 without the
