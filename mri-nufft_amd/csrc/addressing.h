@@ -1,0 +1,46 @@
+// Address arithmetic of the kernels that holds only within limits, as plain
+// functions that the kernels and host checks share.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace hn {
+
+// lines per FFT workgroup: n * L elements held 16 per thread, plus the
+// twiddle table (8 bytes per entry), within 64 KiB of LDS
+constexpr int lines_per_wg(int64_t n, int max_elems) {
+  int L = 16;
+  while (L > 1 && (n * L > max_elems || (size_t)n * (L + 2) * 8 > 65536)) L >>= 1;
+  return L;
+}
+
+// Strided FFT pass.  Position pos of a line of n, column c of its workgroup's
+// adjacent lines, stands at pos * lstride + c cells from the first line's
+// first cell.  Thread (e0, l) of E = threads / L rows takes positions
+// e0 + i * E: slot i.  Of M kept positions (M > 0; hin = M / 2), the e-th
+// stands at e - hin, + n if that is negative.
+
+// every cell of the lines is within 32-bit byte offsets of the first
+constexpr bool strided_fits_32(int64_t n, int64_t lstride, int64_t nx) {
+  return (n * lstride + nx) * 8 < ((int64_t)1 << 32);
+}
+
+// byte offset of position e0, column c
+constexpr uint32_t strided_thread_offset(int e0, int64_t lstride, int c) {
+  return ((uint32_t)e0 * (uint32_t)lstride + (uint32_t)c) * 8u;
+}
+
+// byte offset that slot i adds for every thread (negative ones wrap)
+constexpr uint32_t strided_slot_offset(int i, int E, int hin, int64_t lstride) {
+  return (uint32_t)(i * E - hin) * (uint32_t)lstride * 8u;
+}
+
+// byte offset of the cell that position e = e0 + i * E loads, where the lines
+// fit 32 bits: the terms wrap, their sum is the offset of a cell and does not
+constexpr uint32_t strided_load_offset(uint32_t thread, uint32_t slot, int e, int hin,
+                                       uint32_t line) {
+  return thread + slot + (e < hin ? line : 0u);
+}
+
+}  // namespace hn

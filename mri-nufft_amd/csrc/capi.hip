@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "addressing.h"
 #include "internal.h"
 
 // Partial sums of hipnufft_dot_c64_rows_noalloc: HIPNUFFT_NOALLOC_DOT_ROWS
@@ -128,14 +129,6 @@ std::vector<float> deconv(int64_t M, int64_t nf, int w, double beta) {
     out[i] = (float)(1.0 / (2.0 * s));
   }
   return out;
-}
-
-// lines per FFT workgroup: n * L elements held 16 per thread, plus the
-// twiddle table, within 64 KiB of LDS
-int lines_per_wg(int64_t n, int max_elems) {
-  int L = 16;
-  while (L > 1 && (n * L > max_elems || (size_t)n * (L + 2) * sizeof(float2) > 65536)) L >>= 1;
-  return L;
 }
 
 // allow_direct: a length with other prime factors gets one direct DFT pass

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 
+#include "addressing.h"
 #include "internal.h"
 
 namespace hn {
@@ -829,14 +830,14 @@ __device__ __forceinline__ void store_at(char* base, uint32_t off, float2 v) {
 // - a wave holds 64 / L consecutive positions per slot.  Tiles are at least
 //   that long and aligned (see build_line_masks), so whether a slot counts,
 //   and on which side of the wrap of a kept half it lies, is one scalar
-//   branch per wave, and every address is a scalar base plus one per-thread
-//   offset that all slots share;
+//   branch per wave, and every address is a scalar base plus a 32-bit offset
+//   per thread;
 // - the twiddles are staged behind the lines' loads: before them, they cost
 //   every workgroup a memory latency of its own.
 // 192^3, 16 coils, 3D radial (a ball): both forward passes 3.60 -> 3.22 ms,
 // both backward ones 3.43 -> 2.98; nothing to skip: 256^3 Toeplitz grids,
 // 8 coils, 0.84 -> 0.80 ms, 320^2, 32 coils 116 -> 116 us.
-// HUGE: lines of 4 GiB or more, whose kept positions need 64-bit offsets.
+// HUGE: lines of 4 GiB or more, whose cells need 64-bit offsets.
 template <int S, bool CONV, int EPT, int NT, bool HUGE, int FIX = 0, int FLGL = 0>
 __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
   extern __shared__ float2 buf[];
@@ -876,7 +877,7 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
   const int64_t line0 = (int64_t)t * a.tstride + (int64_t)opos * a.ostride + x0;
   char* lines = reinterpret_cast<char*>(a.data + line0);                // uniform
   const int lc = min(l, a.nx - 1 - x0);  // lanes past the last column repeat it and store nothing
-  const uint32_t v0 = (uint32_t)(e0 * (int)a.lstride + lc) * 8u;        // per thread
+  const uint32_t v0 = strided_thread_offset(e0, a.lstride, lc);         // per thread
   const int hin = a.in_M / 2, hout = a.out_M / 2;
   // slot i of the full side counts
   auto full = [&](int i) {
@@ -898,18 +899,17 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
   // other's loads.  A lane past the last kept position (of a wave's slot that
   // holds some) reads another cell of its line and drops it.
   float2 v[EPT];
-  {
-    const char* p = lines - hin * ls8;
 #pragma unroll
-    for (int i = 0; i < EPT; ++i, p += step8) {
-      const int w0 = wpos + i * E, e = e0 + i * E;
-      v[i] = make_float2(0.f, 0.f);
-      if (a.in_M ? w0 < a.in_M : full(i)) {
-        if constexpr (HUGE)
-          v[i] = *reinterpret_cast<const float2*>(p + (e < hin ? n * ls8 : 0) + v0);
-        else
-          v[i] = load_at(p, v0 + (e < hin ? (uint32_t)(n * ls8) : 0u));
-      }
+  for (int i = 0; i < EPT; ++i) {
+    const int w0 = wpos + i * E, e = e0 + i * E;
+    v[i] = make_float2(0.f, 0.f);
+    if (a.in_M ? w0 < a.in_M : full(i)) {
+      if constexpr (HUGE)
+        v[i] = *reinterpret_cast<const float2*>(
+            lines + (e - hin + (e < hin ? n : 0)) * ls8 + (int64_t)lc * 8);
+      else
+        v[i] = load_at(lines, strided_load_offset(v0, strided_slot_offset(i, E, hin, a.lstride), e,
+                                                  hin, (uint32_t)(n * ls8)));
     }
   }
   // (the twiddles' round trip overlaps the lines')
@@ -1047,7 +1047,7 @@ template <int EPT, int NT, int FIX = 0, int FLGL = 0>
 void launch_strided(bool conv, int sign, dim3 grd, size_t lds, hipStream_t s,
                     const StridedArgs& a) {
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grd, dim3(NT), lds, s, a); };
-  if (((int64_t)a.n * a.lstride + a.nx) * (int64_t)sizeof(float2) < ((int64_t)1 << 32)) {
+  if (strided_fits_32(a.n, a.lstride, a.nx)) {
     if (conv && sign < 0) go(k_fft_strided<-1, true, EPT, NT, false, FIX, FLGL>);
     else if (conv) go(k_fft_strided<1, true, EPT, NT, false, FIX, FLGL>);
     else if (sign < 0) go(k_fft_strided<-1, false, EPT, NT, false, FIX, FLGL>);

@@ -1,0 +1,82 @@
+"""Address arithmetic of the kernels, checked on the host.
+
+The functions of ``csrc/addressing.h`` that the kernels call are compiled with
+the host compiler and walked over every lane and slot, for every fine-grid
+length an axis can have, up to grids of 2^30 cells.
+"""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "mri-nufft_amd", "csrc")
+
+
+def run_check(tmp_path, body):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    src, exe = tmp_path / "check.cpp", tmp_path / "check"
+    src.write_text('#include <algorithm>\n#include <cstdio>\n#include <cstdlib>\n'
+                   '#include "addressing.h"\nusing namespace hn;\n' + body)
+    subprocess.run([cxx, "-O2", "-std=c++17", "-Wall", f"-I{CSRC}",
+                    str(src), "-o", str(exe)], check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
+
+
+STRIDED = r"""
+int main() {
+  long checked = 0;
+  for (int n = 4; n <= 2730; n += 2) {
+    int m = n;
+    for (int p : {2, 3, 5}) while (m % p == 0) m /= p;
+    if (m != 1) continue;
+    const int64_t most = std::min<int64_t>((((int64_t)1 << 30) - 1) / n, 2730 * 2730);
+    const int64_t lim32 = ((int64_t)1 << 29) / n;  // 4 GiB lines
+    for (int64_t ls : {(int64_t)1, (int64_t)n, most / 2, lim32 - 1, lim32, lim32 + 1, most}) {
+      if (ls < 1 || ls > most) continue;
+      for (int64_t nx : {(int64_t)1, std::min<int64_t>(ls, 37), std::min<int64_t>(ls, 2730)})
+        for (int quarter : {0, 1})
+          for (int NT : {256, 512}) {
+            int L = lines_per_wg(n, 8192);
+            if (quarter && (L < 4 || n * ls >= (int64_t)1 << 29)) continue;
+            if (quarter) L /= 4;
+            const int E = NT / L, PW = 64 / L;
+            for (int M : {0, 1, n / 4, n / 3, n / 2 - 1, n / 2, 4 * n / 5, n - 1, n})
+              for (int i = 0; i * E < n; ++i)
+                for (int t = 0; t < NT; t += 1 + (L > 2 && t % L == 0) * (L - 2)) {
+                  const int l = t % L, e0 = t / L, w0 = t / 64 * PW + i * E;
+                  const int e = e0 + i * E, hin = M / 2, lim = M ? M : n;
+                  const int lc = (int)std::min<int64_t>(l, nx - 1);
+                  const uint32_t thread = strided_thread_offset(e0, ls, lc);
+                  // the stores: a uniform base per slot plus the thread's own offset
+                  if (e < n && thread != (uint64_t)(e0 * ls + lc) * 8) {
+                    printf("thread offset: n %d ls %ld L %d e0 %d\n", n, (long)ls, L, e0);
+                    return 1;
+                  }
+                  if (w0 >= lim || !strided_fits_32(n, ls, nx)) continue;
+                  const int64_t off = strided_load_offset(
+                      thread, strided_slot_offset(i, E, hin, ls), e, hin, (uint32_t)(n * ls * 8));
+                  const int64_t pos = e - hin + (e < hin ? n : 0);
+                  ++checked;
+                  if (e < lim && off != (pos * ls + lc) * 8) {
+                    printf("load: n %d M %d ls %ld nx %ld L %d NT %d e %d: %ld\n", n, M, (long)ls,
+                           (long)nx, L, NT, e, (long)off);
+                    return 1;
+                  }
+                }
+          }
+    }
+  }
+  printf("%ld\n", checked);
+  return checked > 1000000 ? 0 : 1;
+}
+"""
+
+
+def test_strided_pass(tmp_path):
+    run_check(tmp_path, STRIDED)
