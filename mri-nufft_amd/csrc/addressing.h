@@ -15,6 +15,15 @@ constexpr int lines_per_wg(int64_t n, int max_elems) {
   return L;
 }
 
+// Lines per workgroup of a pass over `lines` lines: the axis's L, or a
+// quarter of it where that leaves CUs without any workgroup.  A single 2D
+// image has a few dozen workgroups of L lines, whose threads then walk 12 to
+// 16 elements each with most of the chip idle (256^2, one image: the four
+// passes 33.5 -> 21.9 us).  min_l: fewer lines are not allowed (line masks).
+constexpr int lines_of(int L, int64_t lines, int min_l = 1) {
+  return L >= 4 && L / 4 >= min_l && lines < 256 * (int64_t)L ? L / 4 : L;
+}
+
 // Strided FFT pass.  Position pos of a line of n, column c of its workgroup's
 // adjacent lines, stands at pos * lstride + c cells from the first line's
 // first cell.  Thread (e0, l) of E = threads / L rows takes positions
@@ -41,6 +50,13 @@ constexpr uint32_t strided_slot_offset(int i, int E, int hin, int64_t lstride) {
 constexpr uint32_t strided_load_offset(uint32_t thread, uint32_t slot, int e, int hin,
                                        uint32_t line) {
   return thread + slot + (e < hin ? line : 0u);
+}
+
+// bytes from the first cell of `cols` lines to the end of their last.  A wave
+// loads its slot as one, also the lanes past the last position: the loads are
+// bounded by this length, past it they return zero without an access.
+constexpr uint32_t strided_line_bytes(int64_t n, int64_t lstride, int cols) {
+  return (uint32_t)(((n - 1) * lstride + cols) * 8);
 }
 
 }  // namespace hn

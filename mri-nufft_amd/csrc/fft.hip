@@ -831,7 +831,7 @@ __device__ __forceinline__ void store_at(char* base, uint32_t off, float2 v) {
 //   that long and aligned (see build_line_masks), so whether a slot counts,
 //   and on which side of the wrap of a kept half it lies, is one scalar
 //   branch per wave, and every address is a scalar base plus a 32-bit offset
-//   per thread;
+//   per thread; loads are buffer loads bounded by the lines' end;
 // - the twiddles are staged behind the lines' loads: before them, they cost
 //   every workgroup a memory latency of its own.
 // 192^3, 16 coils, 3D radial (a ball): both forward passes 3.60 -> 3.22 ms,
@@ -876,7 +876,8 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
   const int64_t ls8 = a.lstride * (int64_t)sizeof(float2);
   const int64_t line0 = (int64_t)t * a.tstride + (int64_t)opos * a.ostride + x0;
   char* lines = reinterpret_cast<char*>(a.data + line0);                // uniform
-  const int lc = min(l, a.nx - 1 - x0);  // lanes past the last column repeat it and store nothing
+  const int cols = min(L, a.nx - x0);
+  const int lc = min(l, cols - 1);  // lanes past the last column repeat it and store nothing
   const uint32_t v0 = strided_thread_offset(e0, a.lstride, lc);         // per thread
   const int hin = a.in_M / 2, hout = a.out_M / 2;
   // slot i of the full side counts
@@ -896,20 +897,33 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
   // all of a thread's loads are issued before the first LDS store, so they
   // overlap instead of paying one memory latency each.  One code path and no
   // per-thread branch: alternatives for a register would wait for each
-  // other's loads.  A lane past the last kept position (of a wave's slot that
-  // holds some) reads another cell of its line and drops it.
+  // other's loads.  A wave's slot that holds the last position is loaded as
+  // one: its lanes past it load another cell of their lines, or nothing past
+  // the lines' end, and drop it.  (Bounded by the buffer's length the pass
+  // costs less than with each lane's offset clamped: over unbounded loads,
+  // 0.5 against 0.8% of the 128^3 Toeplitz call, 0.1 against 0.3% of the
+  // 192^3, 16-coil adjoint.)
   float2 v[EPT];
+  const int nin = a.in_M ? a.in_M : n;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      lines, (short)0, (int)strided_line_bytes(n, a.lstride, cols), kBufferWord3);
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
     const int w0 = wpos + i * E, e = e0 + i * E;
     v[i] = make_float2(0.f, 0.f);
     if (a.in_M ? w0 < a.in_M : full(i)) {
-      if constexpr (HUGE)
+      if constexpr (HUGE) {
+        const int el = min(e, nin - 1);
         v[i] = *reinterpret_cast<const float2*>(
-            lines + (e - hin + (e < hin ? n : 0)) * ls8 + (int64_t)lc * 8);
-      else
-        v[i] = load_at(lines, strided_load_offset(v0, strided_slot_offset(i, E, hin, a.lstride), e,
-                                                  hin, (uint32_t)(n * ls8)));
+            lines + (el - hin + (el < hin ? n : 0)) * ls8 + (int64_t)lc * 8);
+      } else {
+        v[i] = __builtin_bit_cast(
+            float2, __builtin_amdgcn_raw_buffer_load_b64(
+                        rs,
+                        (int)strided_load_offset(v0, strided_slot_offset(i, E, hin, a.lstride), e,
+                                                 hin, (uint32_t)(n * ls8)),
+                        0, 0));
+      }
     }
   }
   // (the twiddles' round trip overlaps the lines')
@@ -1017,15 +1031,6 @@ int ept_of(int n, int L, int nt = kThreads) {
   return need <= 4 ? 4 : need <= 8 ? 8 : need <= 12 ? 12 : 16;
 }
 
-// Lines per workgroup of a pass over `lines` lines: the axis's L, or a
-// quarter of it where that leaves CUs without any workgroup.  A single 2D
-// image has a few dozen workgroups of L lines, whose threads then walk 12 to
-// 16 elements each with most of the chip idle (256^2, one image: the four
-// passes 33.5 -> 21.9 us).  min_l: fewer lines are not allowed (line masks).
-int lines_of(const FFTAxis& ax, int64_t lines, int min_l = 1) {
-  return ax.L >= 4 && ax.L / 4 >= min_l && lines < 256 * (int64_t)ax.L ? ax.L / 4 : ax.L;
-}
-
 #define HN_EPT_SWITCH(ept, ...)             \
   switch (ept) {                            \
     case 4: { constexpr int EE = 4; __VA_ARGS__ } break;   \
@@ -1094,7 +1099,7 @@ int strided(const hipnufft_plan_s* p, int axis, int T, int in_M, int out_M, int 
     a.ctile_sh = lg2(p->tile[2]);
     a.zero_empty = axis == 1 && out_M != 0;
   }
-  const int L = lines_of(ax, (int64_t)a.nx * a.nouter * T, a.lmask ? 64 / p->tile[axis] : 1);
+  const int L = lines_of(ax.L, (int64_t)a.nx * a.nouter * T, a.lmask ? 64 / p->tile[axis] : 1);
   a.lgL = lg2(L);
   const dim3 grd((unsigned)((a.nx + L - 1) / L), (unsigned)a.nouter, (unsigned)T);
   StageScope timer(p, stage);
@@ -1221,7 +1226,7 @@ int rows_fwd(const hipnufft_plan_s* p, const float2* img, const float2* smaps, i
   a.scale = scale;
   const int rows = a.M0 * a.M1;
   const FFTAxis& ax = p->fft[2];
-  const int L = lines_of(ax, (int64_t)rows * T);
+  const int L = lines_of(ax.L, (int64_t)rows * T);
   a.lgL = lg2(L);
   const dim3 grd((unsigned)((rows + L - 1) / L), (unsigned)T);
   const size_t lds = fft_lds(ax, L);
@@ -1254,7 +1259,7 @@ int rows_adj(const hipnufft_plan_s* p, float2* img, const float2* smaps, int C, 
   const FFTAxis& ax = p->fft[2];
   const int per_img = (smaps ? C : 1) * nmaps;
   const int nimg = (t0 + T - 1) / per_img - t0 / per_img + 1;
-  const int L = lines_of(ax, (int64_t)rows * std::min(T, per_img * nimg));
+  const int L = lines_of(ax.L, (int64_t)rows * std::min(T, per_img * nimg));
   a.lgL = lg2(L);
   // transforms of an image side by side while the rows alone give fewer than
   // two workgroups per CU (each then walks fewer coils)

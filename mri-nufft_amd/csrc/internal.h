@@ -45,6 +45,10 @@ inline bool injected_failure(const char* site) {
                              std::string("kernel launch: ") + hipGetErrorString(e_)); \
   } while (0)
 
+// dword 3 of a raw buffer resource on gfx9-family GPUs (gfx950 included):
+// 32-bit data format, no swizzle, out-of-range offsets return zero
+constexpr int kBufferWord3 = 0x00020000;
+
 constexpr int kMaskWords = 2;       // 64-bit words of a line mask
 constexpr int kMaskTiles = 64 * kMaskWords;
 

@@ -579,7 +579,7 @@ __global__ __launch_bounds__(kMaskTiles) void k_line_masks(const int32_t* ls, in
 // footprints' tile lists, grids of more than kMaskTiles tiles along a strided
 // axis, and tiles that do not hold the adjacent lines of a strided pass
 // along the last axis, or the 64 / lines positions of a wave along its own
-// (what a pass loads must be exactly what spreading has filled).
+// (what a pass takes in must be exactly what spreading has filled).
 static int build_line_masks(hipnufft_plan_s* p) {
   p->prune = 0;
   if (p->sio || p->ndim < 2 || p->nt[0] > kMaskTiles || p->nt[1] > kMaskTiles) return 0;

@@ -98,10 +98,6 @@ struct InterpArgs {
   uint32_t lds_plane_mag;    // LDS row length and plane stride
 };
 
-// dword 3 of a raw buffer resource on gfx9-family GPUs (gfx950 included):
-// 32-bit data format, no swizzle, out-of-range offsets return zero
-constexpr int kBufferWord3 = 0x00020000;
-
 __device__ __forceinline__ int mdiv(int c, uint32_t magic) {
   return (int)__umulhi((uint32_t)c, magic);
 }

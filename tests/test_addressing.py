@@ -40,11 +40,9 @@ int main() {
     for (int64_t ls : {(int64_t)1, (int64_t)n, most / 2, lim32 - 1, lim32, lim32 + 1, most}) {
       if (ls < 1 || ls > most) continue;
       for (int64_t nx : {(int64_t)1, std::min<int64_t>(ls, 37), std::min<int64_t>(ls, 2730)})
-        for (int quarter : {0, 1})
+        // an axis has at least `ls` lines: the pass takes L or, with few of them, a quarter
+        for (int L : {lines_per_wg(n, 8192), lines_of(lines_per_wg(n, 8192), ls)})
           for (int NT : {256, 512}) {
-            int L = lines_per_wg(n, 8192);
-            if (quarter && (L < 4 || n * ls >= (int64_t)1 << 29)) continue;
-            if (quarter) L /= 4;
             const int E = NT / L, PW = 64 / L;
             for (int M : {0, 1, n / 4, n / 3, n / 2 - 1, n / 2, 4 * n / 5, n - 1, n})
               for (int i = 0; i * E < n; ++i)
@@ -59,14 +57,24 @@ int main() {
                     return 1;
                   }
                   if (w0 >= lim || !strided_fits_32(n, ls, nx)) continue;
-                  const int64_t off = strided_load_offset(
-                      thread, strided_slot_offset(i, E, hin, ls), e, hin, (uint32_t)(n * ls * 8));
-                  const int64_t pos = e - hin + (e < hin ? n : 0);
-                  ++checked;
-                  if (e < lim && off != (pos * ls + lc) * 8) {
-                    printf("load: n %d M %d ls %ld nx %ld L %d NT %d e %d: %ld\n", n, M, (long)ls,
-                           (long)nx, L, NT, e, (long)off);
-                    return 1;
+                  // columns of the first and of the last workgroup of a row of nx
+                  for (int cols : {(int)std::min<int64_t>(L, nx), (int)((nx - 1) % L + 1)}) {
+                    const int c = std::min(l, cols - 1);
+                    const int64_t off = strided_load_offset(
+                        strided_thread_offset(e0, ls, c), strided_slot_offset(i, E, hin, ls), e,
+                        hin, (uint32_t)(n * ls * 8));
+                    const int64_t pos = e - hin + (e < hin ? n : 0), end = ((n - 1) * ls + cols) * 8;
+                    const int64_t bytes = strided_line_bytes(n, ls, cols);
+                    ++checked;
+                    // a position's load reads its cell; lanes past the last one
+                    // load, if anything, a cell between the lines' ends
+                    if (bytes != end ||
+                        (e < lim ? off != (pos * ls + c) * 8 || off + 8 > bytes
+                                 : off < bytes && (off < 0 || off % 8 || off + 8 > end))) {
+                      printf("load: n %d M %d ls %ld nx %ld L %d NT %d e %d: %ld\n", n, M, (long)ls,
+                             (long)nx, L, NT, e, (long)off);
+                      return 1;
+                    }
                   }
                 }
           }
