@@ -59,4 +59,23 @@ constexpr uint32_t strided_line_bytes(int64_t n, int64_t lstride, int cols) {
   return (uint32_t)(((n - 1) * lstride + cols) * 8);
 }
 
+// k_interp_pairs: the region's cells from 0, planes apart by a stride, the row
+// table (a cell per region row) behind them.  Before the region, its cells
+// hold the points' weights, kPairWRow floats each (axis 1 at 0, axis 2 at 8).
+constexpr int kStreamRows = 256;  // region rows that row tables hold
+constexpr int kPairNT = 512;
+constexpr int kPairCells = 9216;  // two workgroups per CU
+constexpr int kPairTrips = 2;
+constexpr int kPairPoints = kPairTrips * kPairNT / 8;
+constexpr int kPairWRow = 20;
+constexpr int kPairWeightCells = kPairPoints * kPairWRow / 2;
+
+// cells between the region's planes: at least the plane, 4 modulo 8
+constexpr int pair_plane_stride(int plane) { return plane + ((12 - plane % 8) % 8); }
+
+// the row table's first cell, behind a region of `cells` and the weights
+constexpr int pair_row_table(int cells) {
+  return cells > kPairWeightCells ? cells : kPairWeightCells;
+}
+
 }  // namespace hn

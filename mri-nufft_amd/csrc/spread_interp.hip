@@ -19,6 +19,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "addressing.h"
 #include "internal.h"
 
 namespace hn {
@@ -1685,7 +1686,6 @@ __global__ __launch_bounds__(NT, 4) void k_interp(InterpArgs a) {
 constexpr int kStreamNT = 512;
 constexpr int kStreamNB = 1;
 constexpr int kStreamCells = 9728;
-constexpr int kStreamRows = 256;
 constexpr int kStreamMaxW = 8;
 // 2D regions (32 x 32 tiles plus the halo: 1521 cells) are small, so 2D
 // workgroups of 256 threads hold 2048 cells and several share a CU
@@ -1965,16 +1965,6 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
 // points on 1 to 8 consecutive lanes 3.53 ms, this kernel 2.91 ms.  Of those
 // the set-up takes 0.24; without its gathers the kernel takes 2.47, without
 // its loads 2.27.
-constexpr int kPairNT = 512;
-constexpr int kPairCells = 9216;  // two workgroups per CU
-constexpr int kPairTrips = 2;
-constexpr int kPairPoints = kPairTrips * kPairNT / 8;
-
-// cells between the region's planes: at least the plane, 4 modulo 8
-__host__ __device__ __forceinline__ int pair_plane_stride(int plane) {
-  return plane + ((12 - plane % 8) % 8);
-}
-
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float x) {
   return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
@@ -2041,7 +2031,8 @@ __global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
   const int64_t kstep = a.g.set_off[set + 1] - so;  // k-space offset between transforms
 
   // per region row: wrapped grid offset of its first cell, chunk mask
-  int2* rowtab = reinterpret_cast<int2*>(lds + RCP);
+  // (behind the weights too: the waves write those while others read it)
+  int2* rowtab = reinterpret_cast<int2*>(lds + pair_row_table(RCP));
   for (int r = tid; r < NR; r += NT) {
     const int l0 = mdiv(r, a.rmag[1]);
     const int l1 = r - l0 * R[1];
@@ -2073,8 +2064,7 @@ __global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
   float dens[T];
   // lane s of a point evaluates its weights at cell s; the eight meet in the
   // LDS that the regions take over afterwards
-  constexpr int kWRow = 20;  // floats per point: axis 1 at 0, axis 2 at 8
-  float* wtab = reinterpret_cast<float*>(lds) + (wave * 8 + slot) * kWRow;
+  float* wtab = reinterpret_cast<float*>(lds) + (wave * 8 + slot) * kPairWRow;
 #pragma unroll
   for (int tr = 0; tr < T; ++tr) {
     int ls[3];
@@ -2088,15 +2078,15 @@ __global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
     odd[tr] = ls[2] & 1;
     lbase[tr] = (ls[0] + min(s, W - 1)) * PS + ls[1] * RL + (ls[2] & ~1);
     w0[tr] = wd[0];
-    wtab[tr * (NT / 8) * kWRow + s] = wd[1];
-    wtab[tr * (NT / 8) * kWRow + 8 + s] = wd[2];
+    wtab[tr * (NT / 8) * kPairWRow + s] = wd[1];
+    wtab[tr * (NT / 8) * kPairWRow + 8 + s] = wd[2];
     dens[tr] = (a.mode == 1 && a.density) ? a.density[idx[tr]] : 1.0f;
     kbase[tr] = a.ts * so + (idx[tr] - so);
   }
   __syncthreads();
 #pragma unroll
   for (int tr = 0; tr < T; ++tr) {
-    const float4* wr = reinterpret_cast<const float4*>(wtab + tr * (NT / 8) * kWRow);
+    const float4* wr = reinterpret_cast<const float4*>(wtab + tr * (NT / 8) * kPairWRow);
     const float4 a0 = wr[0], a1 = wr[1], b0 = wr[2], b1 = wr[3];
     const float wy[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
     const float wz[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};

@@ -88,3 +88,25 @@ int main() {
 
 def test_strided_pass(tmp_path):
     run_check(tmp_path, STRIDED)
+
+
+# the row table of every region that the kernel accepts: behind the region and
+# behind the weights, inside the kernel's LDS
+PAIRS = r"""
+int main() {
+  for (int rows = 1; rows <= kStreamRows; ++rows)
+    for (int cells = 128; cells <= kPairCells; cells += 128) {
+      const int t = pair_row_table(cells);
+      if (t < cells || t < kPairWeightCells || t + rows > kPairCells + kStreamRows) {
+        printf("region of %d cells, %d rows: table at %d\n", cells, rows, t);
+        return 1;
+      }
+    }
+  // the weights end where the last point's do
+  return kPairWeightCells * 2 == kPairNT / 64 * 8 * kPairTrips * kPairWRow ? 0 : 1;
+}
+"""
+
+
+def test_interp_pairs_lds(tmp_path):
+    run_check(tmp_path, PAIRS)
