@@ -1784,7 +1784,7 @@ __global__ __launch_bounds__(NT, 4) void k_interp_stream(InterpArgs a) {
     if (c < RC) {
       const int r = mdiv(c, a.lds_row_mag);
       const int z = c - r * RL;
-      if ((rowmask[r] >> ((z + phase) >> 4)) & 1u)
+      if ((rowmask[r] >> (((z + phase) >> 4) & 31)) & 1u)
         off[u] = (uint32_t)(rowoff[r] + wrap_coord(rorg[DL] + z, a.g.nf[DL], a.wrap1)) * 8u +
                  (PAIR ? 0u : 4u * (uint32_t)(pc & 1));
     }
@@ -2038,10 +2038,11 @@ __global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
     const int l1 = r - l0 * R[1];
     rowtab[r] = make_int2((wrap_once(rorg[0] + l0, a.g.nf[0]) * a.g.nf[1] +
                            wrap_once(rorg[1] + l1, a.g.nf[1])) * a.g.nf[2],
-                          a.sub_mask ? (int)a.sub_mask[(int64_t)sub * NR + r] : 0xffff);
+                          a.sub_mask ? (int)a.sub_mask[(int64_t)sub * NR + r] : -1);
   }
   __syncthreads();
-  // chunk of region cell z: (z + phase) / 16 of the row's mask
+  // chunk of region cell z: (z + phase) / 16 of the row's mask (rows of more
+  // than 16 chunks have none: every bit is set)
   const int phase = (rorg[2] & 15) - SH;
   uint32_t off[K];
 #pragma unroll
@@ -2054,7 +2055,7 @@ __global__ __launch_bounds__(kPairNT, 4) void k_interp_pairs(InterpArgs a) {
     const bool in = l0 < R[0] && l1 < R[1];
     const int2 rt = rowtab[in ? l0 * R[1] + l1 : 0];
     const int g = rt.x + wrap_once(rorg[2] - SH + z, a.g.nf[2]);
-    off[u] = in && ((rt.y >> ((z + phase) >> 4)) & 1) ? (uint32_t)g * 8u : kSkip;
+    off[u] = in && ((rt.y >> (((z + phase) >> 4) & 31)) & 1) ? (uint32_t)g * 8u : kSkip;
   }
 
   float wt1[T][W], wt2[T][NC], w0[T];
