@@ -741,7 +741,7 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
   // staged entries that touch it, in list order; a zero record after the
   // staged ones pads the last group of four
   const int zrec = CHUNK * PW;
-  int16_t* lists = reinterpret_cast<int16_t*>(smem + zrec + PW) + wave * BPW * (CHUNK + 4);
+  uint16_t* lists = reinterpret_cast<uint16_t*>(smem + zrec + PW) + wave * BPW * (CHUNK + 4);
   for (int i = (int)threadIdx.x; i < PW; i += 64 * NWAVE) smem[zrec + i] = 0.0f;
   // a lane's operands sit at fixed offsets in a record (block weights, value)
   int ow4[BPW], owy[BPW], owz[BPW];
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
     int ngroups[BPW];
 #pragma unroll
     for (int bi = 0; bi < BPW; ++bi) {
-      int16_t* lst = lists + bi * (CHUNK + 4);
+      uint16_t* lst = lists + bi * (CHUNK + 4);
       int cnt = 0;
       if (bbit[bi]) {  // uniform
         for (int base = 0; base < n; base += 64) {
@@ -781,16 +781,16 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
           const uint64_t bal = __ballot(hit);
           if (hit) lst[cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] =
-              (int16_t)(qi * PW);
+              (uint16_t)(qi * PW);
           cnt += __popcll(bal);
         }
-        if (lane < 4) lst[cnt + lane] = (int16_t)zrec;
+        if (lane < 4) lst[cnt + lane] = (uint16_t)zrec;
       }
       ngroups[bi] = (cnt + 3) >> 2;
     }
 #pragma unroll
     for (int bi = 0; bi < BPW; ++bi) {
-      const int16_t* lst = lists + bi * (CHUNK + 4);
+      const uint16_t* lst = lists + bi * (CHUNK + 4);
       // four entries per step (uniform count); the next step's record offset
       // is read before this step's products
       int o = ngroups[bi] > 0 ? lst[kq] : 0;
@@ -2534,7 +2534,7 @@ int launch_spread_sorted(const hipnufft_plan_s* p, const float2* in, SetRange r,
     a.G = 8;
     const size_t chunk = (size_t)kBlkChunk;
     const size_t lds = sizeof(float) * (chunk + 1) * mfma_record_floats(8, p->tile[1] + p->tile[2]) +
-                       sizeof(int16_t) * 16 * (chunk + 4);
+                       sizeof(uint16_t) * 16 * (chunk + 4);
     if (nitems > 0) {
       const dim3 grd((unsigned)nitems, (unsigned)((r.ts + 7) / 8));
       StageScope timer(p, kStageSpread);
@@ -2593,7 +2593,7 @@ int launch_spread_sorted(const hipnufft_plan_s* p, const float2* in, SetRange r,
     const size_t lds =
         sizeof(float) * (chunk + 1) *  // the records and a zero record
             mfma_record_floats(8 * GH, p->tile[0] + p->tile[1] + p->tile[2]) +
-        sizeof(int16_t) * 16 * (chunk + 4);  // the per-block entry lists
+        sizeof(uint16_t) * 16 * (chunk + 4);  // the per-block entry lists
     if (nitems > 0) {
       const dim3 grd((unsigned)nitems, (unsigned)((r.ts + 8 * GH - 1) / (8 * GH)));
       StageScope timer(p, kStageSpread);
