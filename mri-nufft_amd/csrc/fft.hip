@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "addressing.h"
 #include "internal.h"
@@ -301,9 +302,18 @@ __device__ __forceinline__ void fft_lines_ct(float2* buf, const float2* twl) {
   fft_lines_ct_from<S, EPT, NT, N, LGL, 0>(buf, twl);
 }
 
+// FIX of a kernel whose lines take a runtime plan with a radix-10 pass
+constexpr int kTen = -1;
+
 // All passes of the FFT of the L lines in buf; twl is the twiddle table
 // staged in LDS by stage_twiddles (visible after the caller's barrier).
-template <int S, int EPT, int NT = kThreads>
+// TEN: plans with a radix-10 pass.  Its ten values and their temporaries cost
+// every kernel that holds the case up to 12 VGPRs, whatever its own plan (the
+// adjoint last-axis pass of 300 and 360 points ran at 2 waves per SIMD instead
+// of 3: 150^3, 4 coils 226 us against 163), so only plans that have one take
+// these instances (400 points, 200^3, 4 coils: axis-0 pass 838 us against 930
+// with 2 and 5 apart).
+template <int S, int EPT, int NT = kThreads, bool TEN = false>
 __device__ void fft_lines(float2* buf, const float2* twl, const FFTAxis& ax, int lgL, int LP) {
   int Ns = 1;
   for (int p = 0; p < ax.nrad; ++p) {
@@ -315,7 +325,9 @@ __device__ void fft_lines(float2* buf, const float2* twl, const FFTAxis& ax, int
       case 4: stockham_pass<4, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
       case 5: stockham_pass<5, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
       case 6: stockham_pass<6, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
-      case 10: stockham_pass<10, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
+      case 10:
+        if constexpr (TEN) stockham_pass<10, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl);
+        break;
       default: stockham_pass<8, S, EPT, NT>(buf, ax.n, lgL, LP, Ns, mg, twl); break;
     }
     Ns *= R;
@@ -455,7 +467,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_fwd(RowsArgs a) {
   if constexpr (FIX > 0)
     fft_lines_ct<S, EPT, kThreads, FIX, FLGL>(buf, twl);
   else
-    fft_lines<S, EPT>(buf, twl, a.ax, a.lgL, LP);
+    fft_lines<S, EPT, kThreads, FIX == kTen>(buf, twl, a.ax, a.lgL, LP);
   if (!rok) return;
   float2* g = a.grid + (int64_t)t * a.gstride +
               ((int64_t)kept_pos(i0, a.M0, a.nf0) * a.nf1 + kept_pos(i1, a.M1, a.nf1)) * n;
@@ -546,7 +558,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_adj(RowsArgs a) {
     } else {
       int lg = a.lgL, lp = LP;
       asm volatile("" : "+s"(lg), "+s"(lp));
-      fft_lines<S, EPT>(buf, twl, a.ax, lg, lp);
+      fft_lines<S, EPT, kThreads, FIX == kTen>(buf, twl, a.ax, lg, lp);
     }
     const int rl = rok ? r : 0;  // lanes past the last row read row 0's maps and drop them
     const float2* sm =
@@ -640,13 +652,13 @@ __device__ void dft_lines_direct(float2* buf, const float2* twl, int n, int lgL,
   __syncthreads();
 }
 
-template <int S, int EPT>
+template <int S, int EPT, bool TEN>
 __device__ __forceinline__ void fft_lines_any(float2* buf, const float2* twl, const FFTAxis& ax,
                                               int lgL, int LP) {
   if (ax.direct)
     dft_lines_direct<S, EPT>(buf, twl, ax.n, lgL, LP);
   else
-    fft_lines<S, EPT>(buf, twl, ax, lgL, LP);
+    fft_lines<S, EPT, kThreads, TEN>(buf, twl, ax, lgL, LP);
 }
 
 struct StackArgs {
@@ -668,7 +680,7 @@ struct StackArgs {
 // rows r0 .. r0 + L of transform t: (smap *) image rows -> centred DFT along
 // z -> the NZ sampled positions, written plane-major (L adjacent rows of a
 // plane are one contiguous run)
-template <int EPT>
+template <int EPT, bool TEN>
 __global__ __launch_bounds__(kThreads) void k_stack_fwd(StackArgs a) {
   extern __shared__ float2 buf[];
   const int L = 1 << a.lgL, LP = L + 1;
@@ -704,7 +716,7 @@ __global__ __launch_bounds__(kThreads) void k_stack_fwd(StackArgs a) {
     }
   }
   __syncthreads();
-  fft_lines_any<-1, EPT>(buf, twl, a.ax, a.lgL, LP);
+  fft_lines_any<-1, EPT, TEN>(buf, twl, a.ax, a.lgL, LP);
   // plane-major stores: thread (l, i0) writes planes i0 + q * (kThreads / L)
   const int l = threadIdx.x & (L - 1), i0 = threadIdx.x >> a.lgL;
   const int64_t r = r0 + l;
@@ -719,7 +731,7 @@ __global__ __launch_bounds__(kThreads) void k_stack_fwd(StackArgs a) {
 // rows r0 .. r0 + L of the output image(s) of block y: per transform of the
 // chunk, zero-filled z line from the planes -> centred inverse DFT -> conj
 // smap, summed over the transforms of one image in registers
-template <int EPT>
+template <int EPT, bool TEN>
 __global__ __launch_bounds__(kThreads) void k_stack_adj(StackArgs a) {
   extern __shared__ float2 buf[];
   const int L = 1 << a.lgL, LP = L + 1;
@@ -755,7 +767,7 @@ __global__ __launch_bounds__(kThreads) void k_stack_adj(StackArgs a) {
       buf[j * LP + lq] = (i >= 0 && rq < a.rows) ? pl[(int64_t)i * a.rows] : make_float2(0.f, 0.f);
     }
     __syncthreads();
-    fft_lines_any<1, EPT>(buf, twl, a.ax, a.lgL, LP);
+    fft_lines_any<1, EPT, TEN>(buf, twl, a.ax, a.lgL, LP);
     const float2* sm = a.smaps ? a.smaps + (int64_t)(tt % a.C) * N + rr * Z : nullptr;
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
@@ -957,7 +969,7 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
     if constexpr (FIX > 0)
       fft_lines_ct<S, EPT, NT, FIX, FLGL>(buf, twl);
     else
-      fft_lines<S, EPT, NT>(buf, twl, a.ax, a.lgL, LP);
+      fft_lines<S, EPT, NT, FIX == kTen>(buf, twl, a.ax, a.lgL, LP);
   }
   if constexpr (CONV) {
     const char* kl = reinterpret_cast<const char*>(a.K + (int64_t)opos * a.ostride + x0);
@@ -974,7 +986,7 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
     if constexpr (FIX > 0)
       fft_lines_ct<-S, EPT, NT, FIX, FLGL>(buf, twl);
     else
-      fft_lines<-S, EPT, NT>(buf, twl, a.ax, a.lgL, LP);
+      fft_lines<-S, EPT, NT, FIX == kTen>(buf, twl, a.ax, a.lgL, LP);
   }
   if (!lok) return;
   if (!a.out_M) {
@@ -1023,6 +1035,11 @@ bool fixed_plan(const FFTAxis& ax, int n) {
   return plan_radix(n, p) == 0;
 }
 
+// the axis's runtime plan has a radix-10 pass
+bool has_ten(const FFTAxis& ax) {
+  return std::find(ax.rad, ax.rad + ax.nrad, 10) != ax.rad + ax.nrad;
+}
+
 // complex elements per thread for L lines of n elements: the smallest of 4,
 // 8, 12, 16 with n * L <= EPT * nt (fewer registers, more resident waves for
 // the shorter lines)
@@ -1052,17 +1069,21 @@ template <int EPT, int NT, int FIX = 0, int FLGL = 0>
 void launch_strided(bool conv, int sign, dim3 grd, size_t lds, hipStream_t s,
                     const StridedArgs& a) {
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grd, dim3(NT), lds, s, a); };
-  if (strided_fits_32(a.n, a.lstride, a.nx)) {
-    if (conv && sign < 0) go(k_fft_strided<-1, true, EPT, NT, false, FIX, FLGL>);
-    else if (conv) go(k_fft_strided<1, true, EPT, NT, false, FIX, FLGL>);
-    else if (sign < 0) go(k_fft_strided<-1, false, EPT, NT, false, FIX, FLGL>);
-    else go(k_fft_strided<1, false, EPT, NT, false, FIX, FLGL>);
-  } else {
-    if (conv && sign < 0) go(k_fft_strided<-1, true, EPT, NT, true, FIX, FLGL>);
-    else if (conv) go(k_fft_strided<1, true, EPT, NT, true, FIX, FLGL>);
-    else if (sign < 0) go(k_fft_strided<-1, false, EPT, NT, true, FIX, FLGL>);
-    else go(k_fft_strided<1, false, EPT, NT, true, FIX, FLGL>);
+  // 4 GiB lines have more than 64 positions and are never few: no quarter of
+  // the lines per workgroup, more than 4 elements per thread
+  if constexpr (EPT > 4) {
+    if (!strided_fits_32(a.n, a.lstride, a.nx)) {
+      if (conv && sign < 0) go(k_fft_strided<-1, true, EPT, NT, true, FIX, FLGL>);
+      else if (conv) go(k_fft_strided<1, true, EPT, NT, true, FIX, FLGL>);
+      else if (sign < 0) go(k_fft_strided<-1, false, EPT, NT, true, FIX, FLGL>);
+      else go(k_fft_strided<1, false, EPT, NT, true, FIX, FLGL>);
+      return;
+    }
   }
+  if (conv && sign < 0) go(k_fft_strided<-1, true, EPT, NT, false, FIX, FLGL>);
+  else if (conv) go(k_fft_strided<1, true, EPT, NT, false, FIX, FLGL>);
+  else if (sign < 0) go(k_fft_strided<-1, false, EPT, NT, false, FIX, FLGL>);
+  else go(k_fft_strided<1, false, EPT, NT, false, FIX, FLGL>);
 }
 
 int strided(const hipnufft_plan_s* p, int axis, int T, int in_M, int out_M, int outer_M,
@@ -1127,13 +1148,20 @@ int strided(const hipnufft_plan_s* p, int axis, int T, int in_M, int out_M, int 
   HN_STRIDED_FIXED(192, 4, kThreads, 12)
   HN_STRIDED_FIXED(128, 4, kThreads, 8)
 #undef HN_STRIDED_FIXED
+  const bool ten = has_ten(ax);
   if (ax.n * L > kMaxElemsFFT) {
-    HN_EPT_SWITCH(ept_of(ax.n, L, 2 * kThreads), {
-      launch_strided<EE, 2 * kThreads>(K != nullptr, sign, grd, lds, p->stream, a);
-    });
+    // (more than 8 elements per thread)
+    auto go = [&](auto ept) {
+      constexpr int EE = decltype(ept)::value, NT2 = 2 * kThreads;
+      if (ten) launch_strided<EE, NT2, kTen>(K != nullptr, sign, grd, lds, p->stream, a);
+      else launch_strided<EE, NT2>(K != nullptr, sign, grd, lds, p->stream, a);
+    };
+    if (ept_of(ax.n, L, 2 * kThreads) <= 12) go(std::integral_constant<int, 12>{});
+    else go(std::integral_constant<int, 16>{});
   } else {
     HN_EPT_SWITCH(ept_of(ax.n, L), {
-      launch_strided<EE, kThreads>(K != nullptr, sign, grd, lds, p->stream, a);
+      if (ten) launch_strided<EE, kThreads, kTen>(K != nullptr, sign, grd, lds, p->stream, a);
+      else launch_strided<EE, kThreads>(K != nullptr, sign, grd, lds, p->stream, a);
     });
   }
   HN_LAUNCH_CHECK();
@@ -1206,7 +1234,10 @@ namespace {
   HN_ROWS_FIXED(640, 0, 3)                                                \
   HN_ROWS_FIXED(320, 3, 10)                                               \
   HN_ROWS_FIXED(192, 4, 12)                                               \
-  HN_ROWS_FIXED(128, 4, 8) {                                              \
+  HN_ROWS_FIXED(128, 4, 8)                                                \
+  if (has_ten(ax)) {                                                      \
+    HN_EPT_SWITCH(ept_of(ax.n, L), { HN_ROWS(EE, kTen); });               \
+  } else {                                                                \
     HN_EPT_SWITCH(ept_of(ax.n, L), { HN_ROWS(EE); });                     \
   }
 
@@ -1352,7 +1383,11 @@ int stack_fwd(const StackGeom& g, const float2* img, const float2* smaps, int C,
   a.lgL = lg2(g.ax.L);
   const dim3 grd((unsigned)((g.rows + g.ax.L - 1) / g.ax.L), (unsigned)T);
   HN_EPT_SWITCH(ept_of(g.ax.n, g.ax.L), {
-    hipLaunchKernelGGL((k_stack_fwd<EE>), grd, dim3(kThreads), fft_lds(g.ax), s, a);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grd, dim3(kThreads), fft_lds(g.ax), s, a);
+    };
+    if (has_ten(g.ax)) go(k_stack_fwd<EE, true>);
+    else go(k_stack_fwd<EE, false>);
   });
   HN_LAUNCH_CHECK();
   return 0;
@@ -1377,7 +1412,11 @@ int stack_adj(const StackGeom& g, const float2* planes, const float2* smaps, int
   const int nimg = smaps ? ((t0 + T - 1) / C - t0 / C + 1) : T;
   const dim3 grd((unsigned)((g.rows + g.ax.L - 1) / g.ax.L), (unsigned)nimg);
   HN_EPT_SWITCH(ept_of(g.ax.n, g.ax.L), {
-    hipLaunchKernelGGL((k_stack_adj<EE>), grd, dim3(kThreads), fft_lds(g.ax), s, a);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grd, dim3(kThreads), fft_lds(g.ax), s, a);
+    };
+    if (has_ten(g.ax)) go(k_stack_adj<EE, true>);
+    else go(k_stack_adj<EE, false>);
   });
   HN_LAUNCH_CHECK();
   return 0;

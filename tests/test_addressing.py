@@ -39,7 +39,16 @@ int main() {
     const int64_t lim32 = ((int64_t)1 << 29) / n;  // 4 GiB lines
     for (int64_t ls : {(int64_t)1, (int64_t)n, most / 2, lim32 - 1, lim32, lim32 + 1, most}) {
       if (ls < 1 || ls > most) continue;
-      for (int64_t nx : {(int64_t)1, std::min<int64_t>(ls, 37), std::min<int64_t>(ls, 2730)})
+      for (int64_t nx : {(int64_t)1, std::min<int64_t>(ls, 37), std::min<int64_t>(ls, 2730)}) {
+        {
+          // lines past 32 bits: all of the axis's lines per workgroup, more than
+          // 4 elements per thread (the only forms with 64-bit offsets)
+          const int L = lines_per_wg(n, 8192), NT = n * L > 4096 ? 512 : 256;
+          if (!strided_fits_32(n, ls, nx) && (lines_of(L, ls) != L || n * L <= 4 * NT)) {
+            printf("64-bit lines: n %d ls %ld\n", n, (long)ls);
+            return 1;
+          }
+        }
         // an axis has at least `ls` lines: the pass takes L or, with few of them, a quarter
         for (int L : {lines_per_wg(n, 8192), lines_of(lines_per_wg(n, 8192), ls)})
           for (int NT : {256, 512}) {
@@ -78,6 +87,7 @@ int main() {
                   }
                 }
           }
+      }
     }
   }
   printf("%ld\n", checked);
