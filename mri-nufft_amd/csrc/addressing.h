@@ -35,7 +35,8 @@ constexpr bool strided_fits_32(int64_t n, int64_t lstride, int64_t nx) {
   return (n * lstride + nx) * 8 < ((int64_t)1 << 32);
 }
 
-// byte offset of position e0, column c
+// byte offset of position e0, column c (right for every cell of lines that
+// fit 32 bits, and for the threads' first positions of any)
 constexpr uint32_t strided_thread_offset(int e0, int64_t lstride, int c) {
   return ((uint32_t)e0 * (uint32_t)lstride + (uint32_t)c) * 8u;
 }
@@ -45,9 +46,9 @@ constexpr uint32_t strided_slot_offset(int i, int E, int hin, int64_t lstride) {
   return (uint32_t)(i * E - hin) * (uint32_t)lstride * 8u;
 }
 
-// byte offset of the cell that position e = e0 + i * E loads, where the lines
-// fit 32 bits: the terms wrap, their sum is the offset of a cell and does not
-constexpr uint32_t strided_load_offset(uint32_t thread, uint32_t slot, int e, int hin,
+// byte offset of the cell of position e = e0 + i * E, where the lines fit 32
+// bits: the terms wrap, their sum is the offset of a cell and does not
+constexpr uint32_t strided_cell_offset(uint32_t thread, uint32_t slot, int e, int hin,
                                        uint32_t line) {
   return thread + slot + (e < hin ? line : 0u);
 }

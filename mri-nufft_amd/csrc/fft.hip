@@ -932,7 +932,7 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
         v[i] = __builtin_bit_cast(
             float2, __builtin_amdgcn_raw_buffer_load_b64(
                         rs,
-                        (int)strided_load_offset(v0, strided_slot_offset(i, E, hin, a.lstride), e,
+                        (int)strided_cell_offset(v0, strided_slot_offset(i, E, hin, a.lstride), e,
                                                  hin, (uint32_t)(n * ls8)),
                         0, 0));
       }
@@ -1005,13 +1005,20 @@ __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {
                  buf[q0 + (i * E - hout + (w0 < hout ? n : 0)) * LP]);
     }
   } else {
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) {
-      const int e = e0 + i * E;
-      if (e < a.out_M) {
-        const int pos = e - hout + (e < hout ? n : 0);
+    // A kept half that is no multiple of a wave's positions.  A loop, not
+    // unrolled: a dozen copies of it cost the other forms their place in the
+    // instruction cache (192^3, 16 coils, which never come here: axis-0 pass
+    // 1.99 -> 1.85 ms forward, 1.89 -> 1.77 adjoint).  32-bit offsets where the
+    // length is not fixed (150^3, 4 coils, axis 0: 437 us with 64, 418); in the
+    // fixed-length kernels they changed the other forms for the worse (1.85 ->
+    // 2.02), and 64 bits cost them nothing here (126^3: 153 us either way).
+#pragma unroll 1
+    for (int e = e0; e < a.out_M; e += E) {
+      const int pos = e - hout + (e < hout ? n : 0);
+      if constexpr (HUGE || FIX > 0)
         *reinterpret_cast<float2*>(lines + (int64_t)pos * ls8 + 8 * l) = buf[pos * LP + l];
-      }
+      else
+        store_at(lines, strided_thread_offset(pos, a.lstride, lc), buf[pos * LP + l]);
     }
   }
 }

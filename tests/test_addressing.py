@@ -69,12 +69,17 @@ int main() {
                   // columns of the first and of the last workgroup of a row of nx
                   for (int cols : {(int)std::min<int64_t>(L, nx), (int)((nx - 1) % L + 1)}) {
                     const int c = std::min(l, cols - 1);
-                    const int64_t off = strided_load_offset(
+                    const int64_t off = strided_cell_offset(
                         strided_thread_offset(e0, ls, c), strided_slot_offset(i, E, hin, ls), e,
                         hin, (uint32_t)(n * ls * 8));
                     const int64_t pos = e - hin + (e < hin ? n : 0), end = ((n - 1) * ls + cols) * 8;
                     const int64_t bytes = strided_line_bytes(n, ls, cols);
                     ++checked;
+                    // a store of the cell at pos by its own offset
+                    if (e < lim && strided_thread_offset((int)pos, ls, c) != (pos * ls + c) * 8) {
+                      printf("store: n %d M %d ls %ld e %d\n", n, M, (long)ls, e);
+                      return 1;
+                    }
                     // a position's load reads its cell; lanes past the last one
                     // load, if anything, a cell between the lines' ends
                     if (bytes != end ||
