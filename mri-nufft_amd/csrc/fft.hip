@@ -847,8 +847,9 @@ __device__ __forceinline__ void store_at(char* base, uint32_t off, float2 v) {
 // - the twiddles are staged behind the lines' loads: before them, they cost
 //   every workgroup a memory latency of its own.
 // 192^3, 16 coils, 3D radial (a ball): both forward passes 3.60 -> 3.22 ms,
-// both backward ones 3.43 -> 2.98; nothing to skip: 256^3 Toeplitz grids,
-// 8 coils, 0.84 -> 0.80 ms, 320^2, 32 coils 116 -> 116 us.
+// both backward ones 3.43 -> 2.98 (2.90 and 2.78 with the kept halves' loop at
+// the end rolled); nothing to skip: 256^3 Toeplitz grids, 8 coils, 0.84 ->
+// 0.80 ms, 320^2, 32 coils 116 -> 116 us.
 // HUGE: lines of 4 GiB or more, whose cells need 64-bit offsets.
 template <int S, bool CONV, int EPT, int NT, bool HUGE, int FIX = 0, int FLGL = 0>
 __global__ __launch_bounds__(NT) void k_fft_strided(StridedArgs a) {

@@ -878,9 +878,10 @@ __global__ __launch_bounds__(64 * NWAVE, 4 / GH) void k_spread_mfma(SpreadArgs a
   }
 }
 
-// Record of an entry for the few-transform matrix kernel: as
-// write_mfma_entry (GT strengths, each axis's weight at every tile cell),
-// with the touched-block mask over blocks of 4 x 4 x ZB cells.
+// Record of an entry for the few-transform matrix kernel at sp: one mask of
+// the blocks of 4 x 4 x ZB cells that its footprint meets (bit (b0 nb1 + b1)
+// nb2 + b2), GT strengths and, per axis, the weight of every tile cell along
+// it, as in the records of write_mfma_half.
 template <int GT, int ZB>
 __device__ __forceinline__ void write_mfmaz_entry(float* sp, const BlkPos& r,
                                                   const SpreadArgs& a, int t0, int Gv,
